@@ -11,10 +11,20 @@ FLAGS=(-O3 -std=c++17 -fPIC --offload-arch="$ARCH" -ffp-contract=off -fno-gpu-fl
        -Xclang -target-feature -Xclang -packed-fp32-ops
        -I"$root/include" -I"$here/csrc")
 mkdir -p "$here/_build"
-hipcc "${FLAGS[@]}" ${CGFD_EXTRA_FLAGS:-} -c "$here/csrc/cgfd_kernels.hip" -o "$here/_build/cgfd_kernels.o"
-hipcc "${FLAGS[@]}" -c "$here/csrc/cgfd_capi.hip" -o "$here/_build/cgfd_capi.o"
+# the kernels in nine parts (see CGFD_STAGE_TU), side by side
+objs=()
+pids=()
+for tu in 1 2 3 4 5 6 7 8 0; do
+    hipcc "${FLAGS[@]}" ${CGFD_EXTRA_FLAGS:-} -DCGFD_STAGE_TU=$tu -c "$here/csrc/cgfd_kernels.hip" \
+        -o "$here/_build/cgfd_kernels$tu.o" &
+    pids+=($!)
+    objs+=("$here/_build/cgfd_kernels$tu.o")
+done
+hipcc "${FLAGS[@]}" -c "$here/csrc/cgfd_capi.hip" -o "$here/_build/cgfd_capi.o" &
+pids+=($!)
+for p in "${pids[@]}"; do wait "$p"; done
 g++ -O2 -std=c++17 -fPIC -ffp-contract=off -Wall -I"$root/include" -c "$here/csrc/cgfd_ncio.cpp" -o "$here/_build/cgfd_ncio.o"
-hipcc -shared -fPIC --offload-arch="$ARCH" -o "$here/libcgfd3d.so.tmp" "$here/_build/cgfd_kernels.o" "$here/_build/cgfd_capi.o" \
+hipcc -shared -fPIC --offload-arch="$ARCH" -o "$here/libcgfd3d.so.tmp" "${objs[@]}" "$here/_build/cgfd_capi.o" \
       "$here/_build/cgfd_ncio.o"
 mv -f "$here/libcgfd3d.so.tmp" "$here/libcgfd3d.so"
 echo "built $here/libcgfd3d.so"

@@ -108,9 +108,9 @@ struct cgfd_ctx {
     hipGraphExec_t gexec[4] = {nullptr, nullptr, nullptr, nullptr};
     int rows = 4, zchunks = 1;
     bool zc_tuned = false; // zchunks chosen by cgfd_autotune or cgfd_set_tuning: fused batches keep it
-    int tile_w = 0;        // LDS kernel tile width set by cgfd_set_tile_width (0: none)
+    int tile_w = 0;        // tile width set by cgfd_set_tile_width (0: none)
     int tile_pref = 0;     // the width cgfd_autotune found faster than the default (0: none)
-    int variant = 0; // stage kernel: 0 = LDS-staged planes, 1 = direct loads
+    int variant = 0; // stage kernel: 0 = half-system workgroups, 1 = direct loads, 2 = split
     char *args_d = nullptr; // argument image (kCtxArgBytes: stage, traction-image and trace blocks)
     bool args_dirty = true;
     // batches led by this context (the first of cgfd_run_batch's list):
@@ -221,7 +221,7 @@ static void fb_signs(int t, int k, int *sx, int *sz)
 // planes, 5.59 ms with 10 of 30; with later kernels 5.338 ms at 10 chunks,
 // 5.328 at 12, 5.305 at 15, 5.300 at 20 and 5.313 at 25; 200x200x150 is
 // fastest at 12 chunks of 13 planes).
-// Tile width of the LDS stage kernel: the one set or tuned, else 32 when a
+// Tile width of the default stage kernel: the one set or tuned, else 32 when a
 // row of ni cells takes over 8 % more lanes in 64-column tiles than in
 // 32-column ones.  Measured per stage: 80 cells (128 vs 96 lanes) 13 % and
 // 200 cells (256 vs 224) 10 % faster at 32; 600 cells (640 vs 608) 0.5 %
@@ -236,7 +236,7 @@ static int tile_width(const cgfd_ctx *c)
     return narrow_pays((c->g.ni + 63) / 64 * 64, (c->g.ni + 31) / 32 * 32) ? 32 : 64;
 }
 
-// LDS-kernel tiles of one z plane at tile width tw
+// tiles of one z plane at tile width tw
 static long plane_tiles(const cgfd_ctx *c, int tw)
 {
     const int tr = stage_tile_rows(c->prec == CGFD_FP64, tw);
@@ -1231,7 +1231,7 @@ int cgfd_set_graph(cgfd_ctx *c, int on)
 } // extern "C"
 
 // A batch runs as one launch per kernel when its grids share a device, the
-// precision, the LDS stage variant with the same metric mode, and the step
+// precision, the default stage variant with the same metric mode, and the step
 // phase currT % 4 (which fixes the forward/backward pattern of every
 // stage), and no context is timing its kernels.  Grid sizes may differ.
 
@@ -1275,8 +1275,7 @@ static void batch_layout(cgfd_ctx *const *ctxs, int n, int tw, int *zlen, int *s
     for (int i = 0; i < n; i++) {
         const int nk = ctxs[i]->g.nk;
         const int zci = ctxs[i]->zc_tuned ? std::max(1, std::min(ctxs[i]->zchunks, nk))
-                                          : (int)std::min(std::max(zc, (long)(nk + CGFD_BATCH_PLANES - 1) /
-                                                                              CGFD_BATCH_PLANES),
+                                          : (int)std::min(std::max(zc, (long)(nk + CGFD_BATCH_PLANES - 1) / CGFD_BATCH_PLANES),
                                                           (long)std::max(1, nk / 2));
         zlen[i] = (nk + zci - 1) / zci;
         starts[i + 1] = starts[i] + (int)(plane_tiles(ctxs[i], tw) * zci);
@@ -1598,7 +1597,7 @@ int cgfd_autotune(cgfd_ctx *c, int trial_steps, int *chosen)
     c->zchunks = best;
     c->zc_tuned = true;
     c->args_dirty = true;
-    // then the LDS kernel's other tile width (FP32) at those chunks, unless
+    // then the other tile width (FP32) at those chunks, unless
     // cgfd_set_tile_width fixed one
     if (!rc && c->prec == CGFD_FP32 && c->variant == 0 && c->tile_w == 0) {
         c->tile_pref = tile_width(c) == 64 ? 32 : 64;
@@ -1951,7 +1950,7 @@ int cgfd_set_variant(cgfd_ctx *c, int variant)
 {
     if (!c) return CGFD_EINVAL;
     if (variant < 0 || variant > 2)
-        return fail(c, CGFD_EINVAL, "variant must be 0 (LDS), 1 (direct) or 2 (split velocity/stress)");
+        return fail(c, CGFD_EINVAL, "variant must be 0 (default), 1 (direct) or 2 (split velocity/stress)");
     if (variant != c->variant) {
         c->variant = variant;
         // captured cycles launch the old variant's kernels: the next run

@@ -42,7 +42,7 @@ template <typename R> struct StageArgs {
     int zlen;
     int hmet; // 1: horizontal metrics are the constants 1/0 (variant 0 loads only the zeta metrics)
     int zcon; // hybrid grid: planes z < zcon take the Cartesian contraction (0: none)
-    int tile; // LDS kernel tile width, 64 or 32 columns (host side: picks the kernel)
+    int tile; // default stage kernel's tile width, 64 or 32 columns (host side: picks the kernel)
     const int *step; // device step counter: the current step currT (Tindex = 2*currT + tinc)
 };
 
@@ -81,7 +81,7 @@ constexpr int kRecArgsOffset = kTimgArgsOffset + 4 * kTimgArgsBytes;
 constexpr int kCtxArgBytes = 8192;
 static_assert(kRecArgsOffset + kRecArgsBytes <= kCtxArgBytes, "argument image too small");
 
-// variant 0: LDS-staged xy planes (default); 1: direct loads of the in-plane
+// variant 0: half-system workgroups (default); 1: direct loads of the in-plane
 // taps; 2: split velocity/stress kernels.  `a` is the host copy of the
 // argument block (launch geometry), `pa` the same block in device memory,
 // read by the kernel.  tinc = 0, 1, 1, 2 in stages 0-3: the kernel forms
@@ -89,13 +89,13 @@ static_assert(kRecArgsOffset + kRecArgsBytes <= kCtxArgBytes, "argument image to
 template <typename R>
 void launch_stage(int variant, int sx, int sz, int st, const StageArgs<R> &a, const StageArgs<R> *pa, int tinc,
                   int rows, int zchunks, hipStream_t s);
-// The same stage of nctx grids in one launch of the LDS variant: grid c's
-// argument block lies c * kCtxArgBytes after pa and it owns workgroups
-// starts[c] .. starts[c+1]-1 (starts in device memory, starts[nctx] =
+// The same stage of nctx grids in one launch of the default variant: grid c's
+// argument block lies c * kCtxArgBytes after pa and it owns tiles (two
+// workgroups each) starts[c] .. starts[c+1]-1 (starts in device memory, starts[nctx] =
 // nblocks); all grids share the step phase and the metric mode hmet.
 // nctx = -n: n grids of one size and z-chunk length on one medium, the n
 // copies of each tile run one after another on one XCD (starts unused).
-// rows of an LDS stage-kernel tile of tw columns (64 or 32; FP64 runs 64)
+// rows of a default stage-kernel tile of tw columns (64 or 32; FP64 runs 64)
 int stage_tile_rows(bool fp64, int tw);
 template <typename R>
 void launch_stage_batch(int sx, int sz, int st, int hmet, int hybrid, int tw, const StageArgs<R> *pa,

@@ -17,12 +17,9 @@
 //                 stage.  The reference's 27 derivative arrays, its rate
 //                 arrays and its per-stage state copies never exist.
 //
-// stage_kernel mapping: a 64-lane wavefront owns 64 consecutive x of one
-// (y) row; a workgroup stacks `rows` such rows; blockIdx.z picks a chunk of
-// z planes that each lane sweeps upward.  The z-direction stencil taps live
-// in a 5-deep register window per component, so each plane of the stage
-// input is fetched from memory once by its own lane; x and y taps are read
-// from neighbouring lanes' lines through the vector L1/L2.
+// The default stage kernel (stage_half_kernel) gives every tile of columns two
+// workgroups, one for the velocity half of the system and one for the stress
+// half; stage_direct_kernel and stage_split_kernel are the cross-checks.
 #include "cgfd_kernels.h"
 
 namespace cgfd {
@@ -597,7 +594,7 @@ __device__ __forceinline__ void finish_cell(AP a, const Column<R> &k, const Cell
     pgv_update<R, ST>(a, k, in, hv, z - (geom_of(a).nk - 3));
 }
 
-// Variant "direct": the x and y stencil taps are read straight from memory
+// Variant "direct" (cross-check): the x and y stencil taps are read straight from memory
 // (vector L1/L2); one lane per (x,y) column sweeps its z chunk with the z taps
 // in a 5-deep register window.
 template <typename R, int SX, int SZ, int ST>
@@ -664,55 +661,590 @@ __global__ void __launch_bounds__(256) stage_direct_kernel(const StageArgs<R> *p
     }
 }
 
-// Variant "lds": xy-plane staging.  A workgroup of LDS_TY wavefronts owns a
-// 64 x LDS_TY (or 32 x 2*LDS_TY) tile of (x,y) columns and sweeps a chunk of
-// z planes.  Per plane
-// every lane writes its cell of the 9 stage-input components into an LDS tile
-// that also holds the one-sided halo (1 cell behind and 3 ahead for forward
-// differences, 3 behind and 1 ahead for backward), so all 18 in-plane stencils
-// of a cell are LDS reads at immediate offsets from one address.  The z taps
-// stay in the per-lane 5-deep register window; the next plane's global loads
-// (window lead and halo) are issued before the current plane's arithmetic,
-// unconditionally (lanes outside the grid read a clamped in-bounds address
-// and discard the value), so no branch splits the load stream.  A plane's
-// halo is fetched together with its window lead and parked in an LDS ring
-// until the plane is the centre (see below).
-#ifndef CGFD_LDS_TY
-#define CGFD_LDS_TY 4
-#endif
-constexpr int LDS_TY = CGFD_LDS_TY;
-static_assert(LDS_TY >= 4 && LDS_TY <= 16 && 4 * LDS_TY <= 64, "x-halo lanes must fit one wavefront");
-// FP64 keeps 4-row tiles: its one wavefront per SIMD needs the full register file
-template <typename R> constexpr int lds_ty() { return sizeof(R) == 4 ? LDS_TY : 4; }
-#ifndef CGFD_LDS_WAVES
-#define CGFD_LDS_WAVES 2
-#endif
-#ifndef CGFD_HALO_RING
-#define CGFD_HALO_RING 1
-#endif
-#define CGFD_LDS_ATTR __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? CGFD_LDS_WAVES : 1, 8)))
+// ---------------------------------------------------------------------------
+// half-system stage kernel (the default)
+// ---------------------------------------------------------------------------
+// Bound by HBM on large grids (51 streams in stages 1-2, which a plain copy of
+// that many streams moves at 5.1-5.4 TB/s) and by the latency of one
+// wavefront's instructions on small ones; no matrix product in it.
+//
+// A workgroup of HALF_TY wavefronts owns a 64 x 4 (or 32 x 8) tile of columns
+// and sweeps a chunk of z planes.  The z taps live in a 5-deep register window
+// per component; each plane's stencil inputs, with the one-sided halo (1 cell
+// behind and 3 ahead for forward differences, 3 and 1 for backward), are staged
+// in LDS, so the in-plane taps are LDS reads at immediate offsets.  The next
+// plane's window lead and halo are loaded before the current plane's
+// arithmetic, without a branch: a skippable load would make the compiler's
+// wait counts assume the path that skips it.
+//
+// Why two workgroups per tile and not one cell per lane: a lane that advances
+// all nine components needs 256 registers (2 wavefronts per SIMD in FP32, 1 in
+// FP64); half the components need 124-134 (FP64: 254), so 4 and 2 fit, each
+// wavefront has half as long a chain of instructions per plane, and a small
+// grid has twice the workgroups.  What is read twice, the metrics and in stage
+// 0 the step-start field, is read by the partner at about the same time.
+// Stage kernel, one cell per lane -> two halves: 600x600x300 5.31 -> 5.15 ms,
+// 200x200x150 428 -> 411 us, 149x131x97 with all nine metrics 171 -> 150 us,
+// 160x144x96 FP64 415 -> 313 us, 64x64x64 31.3 -> 27.8 us, 40x32x20 20.5 ->
+// 15.4 us.  Measured and not taken: both halves in one workgroup of 8
+// wavefronts that share the tile (5.24 ms, 160 us: each plane waits for the
+// slower half), the absorbing operands loaded ahead of the stencil (its
+// registers cost a wavefront per SIMD), the tiles of odd stages in reverse
+// order (5.31 ms), a wait for the previous plane's stores (5.33 ms).
+// The half of the system a workgroup advances.  PART 0 (velocity): the 18
+// derivatives of the six stresses, the momentum rates, traction-image override
+// and point forces; writes Vx Vy Vz.  PART 1 (stress): the 9 derivatives of
+// the velocities with the free-surface closure, Hooke's law, moment sources;
+// writes the six stresses.
+template <int PART> struct Half {
+    static constexpr int NIN = PART == 0 ? 6 : 3;     // stencil inputs
+    static constexpr int I0 = PART == 0 ? TXX : VX;   // first of them
+    static constexpr int NO = PART == 0 ? 3 : 6;      // outputs
+    static constexpr int O0 = PART == 0 ? VX : TXX;   // first of them
+};
 
-template <typename R, int SX, int SZ, int ST, int HM, int TW>
-__global__ void __launch_bounds__(64 * lds_ty<R>()) CGFD_LDS_ATTR
-stage_lds_kernel(const StageArgs<R> *pa, const int *starts, int nctx, int tinc)
+template <typename R, int PART> struct HalfIn {
+    R med[2]; // PART 0: 1/rho; PART 1: lam2mu, miu
+    R m[9];
+    R fw[Half<PART>::NO], tw[Half<PART>::NO];
+};
+
+template <typename R, int ST, int HM, int PART, typename AP>
+__device__ __forceinline__ void load_half(AP a, unsigned pb, long fs, HalfIn<R, PART> &in)
 {
-    // The argument block lives in device memory and is read through the
-    // constant address space, so fields are fetched with scalar loads where
-    // they are used instead of being preloaded into (and spilled from) SGPRs.
-    // A batched launch (nctx > 1) covers several grids: grid c owns
-    // workgroups starts[c] .. starts[c+1]-1 and its block lies c *
-    // kCtxArgBytes after pa.  The search runs on scalar registers.  With
-    // nctx = -n the n grids are identical and interleaved tile by tile.
+    constexpr int NO = Half<PART>::NO, O0 = Half<PART>::O0;
+    if (PART == 0) {
+        in.med[0] = ldg_once(a->med + 2 * fs, pb);
+    } else {
+        in.med[0] = ldg_once(a->med, pb);
+        in.med[1] = ldg_once(a->med + fs, pb);
+    }
+    if (HM) {
+        in.m[XIX] = in.m[ETY] = (R)1;
+        in.m[XIY] = in.m[XIZ] = in.m[ETX] = in.m[ETZ] = (R)0;
+#pragma unroll
+        for (int m = ZTX; m <= ZTZ; ++m) in.m[m] = ldg(a->met + m * fs, pb);
+    } else {
+#pragma unroll
+        for (int m = 0; m < 9; ++m) in.m[m] = ldg(a->met + m * fs, pb);
+    }
+#pragma unroll
+    for (int c = 0; c < NO; ++c) {
+        if (ST <= 2) in.fw[c] = ST == 0 ? ldg(a->win + (O0 + c) * fs, pb) : ldg_once(a->fw + (O0 + c) * fs, pb);
+        if (ST >= 1) in.tw[c] = ldg_once((const R *)a->tw + (O0 + c) * fs, pb);
+    }
+}
+
+template <typename R, int PART> struct HalfAux {
+    R ai[Half<PART>::NO], af[Half<PART>::NO], at[Half<PART>::NO];
+};
+
+template <typename R, int ST, int PART, typename AP>
+__device__ __forceinline__ void load_half_aux(AP a, int ax, long aidx, HalfAux<R, PART> &v)
+{
+    const long as = a->astr[ax];
+    const unsigned off = (unsigned)(aidx * (long)sizeof(R));
+#pragma unroll
+    for (int i = 0; i < Half<PART>::NO; ++i) {
+        const long o = (Half<PART>::O0 + i) * as;
+        v.ai[i] = ldg_once(a->ain[ax] + o, off);
+        if (ST == 1 || ST == 2) v.af[i] = ldg_once(a->af[ax] + o, off);
+        if (ST >= 1) v.at[i] = ldg_once((const R *)a->at[ax] + o, off);
+    }
+}
+
+template <typename R, int ST, int PART, typename AP>
+__device__ __forceinline__ void store_half_aux(AP a, int ax, long aidx, const HalfAux<R, PART> &v,
+                                               const R (&ha)[Half<PART>::NO])
+{
+    const long as = a->astr[ax];
+    const unsigned off = (unsigned)(aidx * (long)sizeof(R));
+#pragma unroll
+    for (int i = 0; i < Half<PART>::NO; ++i) {
+        R *ao = a->aout[ax] + (Half<PART>::O0 + i) * as;
+        R *at = a->at[ax] + (Half<PART>::O0 + i) * as;
+        if (ST == 0) {
+            stg_once(ao, off, v.ai[i] + a->alpha * ha[i]);
+            stg_once(at, off, v.ai[i] + a->beta * ha[i]);
+        } else if (ST < 3) {
+            stg_once(ao, off, v.af[i] + a->alpha * ha[i]);
+            stg_once(at, off, v.at[i] + a->beta * ha[i]);
+        } else {
+            stg_once(ao, off, v.at[i] + a->beta * ha[i]);
+        }
+    }
+}
+
+// hv[c] -= ai/B, ha = D*DB - APD*ai of one axis
+template <typename R, int PART>
+__device__ __forceinline__ void aux_rates(const R (&D)[Half<PART>::NO], const HalfAux<R, PART> &v, R B, R DB, R APD,
+                                          R (&hv)[Half<PART>::NO], R (&ha)[Half<PART>::NO])
+{
+#pragma unroll
+    for (int c = 0; c < Half<PART>::NO; ++c) {
+        hv[c] -= v.ai[c] / B;
+        ha[c] = D[c] * DB - APD * v.ai[c];
+    }
+}
+
+template <typename R> __device__ __forceinline__ void surface_stress(R s, R lam2mu, R lambda, R miu, const R (&m)[9], R d1, R d2, R d3, R (&ha)[6])
+{
+    const R ztx = m[ZTX], zty = m[ZTY], ztz = m[ZTZ];
+    ha[0] += s * (lam2mu * ztx * d1 + lambda * zty * d2 + lambda * ztz * d3);
+    ha[1] += s * (lambda * ztx * d1 + lam2mu * zty * d2 + lambda * ztz * d3);
+    ha[2] += s * (lambda * ztx * d1 + lambda * zty * d2 + lam2mu * ztz * d3);
+    ha[3] += s * (zty * d1 + ztx * d2) * miu;
+    ha[4] += s * (ztz * d1 + ztx * d3) * miu;
+    ha[5] += s * (ztz * d2 + zty * d3) * miu;
+}
+
+// What a lane keeps of its column between planes: its absorbing factors (read
+// again in each plane, they would put a dependent load in front of every
+// absorbing cell's divisions).
+template <typename R> struct HalfCol {
+    bool inx, iny; // inside an x or y absorbing layer
+    R APDx, Bx, DBx, APDy, By, DBy;
+};
+
+// rates of one cell's half (see cell_rates for the reference citations)
+template <typename R, int SX, int SZ, int ST, int HY, int PART, typename AP>
+__device__ __forceinline__ void half_rates(AP a, const HalfCol<R> &k, const HalfIn<R, PART> &in,
+                                           R (&Dx)[Half<PART>::NIN], R (&Dy)[Half<PART>::NIN],
+                                           R (&Dz)[Half<PART>::NIN], const R (&w)[Half<PART>::NIN][5], int x, int y,
+                                           int z, int &e, int tindex, R (&hv)[Half<PART>::NO])
+{
+    constexpr int NO = Half<PART>::NO;
+    const Geom g = geom_of(a);
+    const int top = z - (g.nk - 3);
+    const unsigned cxy = (unsigned)(y * g.nxp + x); // offset of the column inside one [nj][nxp] map
+    const R *pmz = a->pml + 3 * g.ni + 3 * g.nj;
+    const R xix = in.m[XIX], xiy = in.m[XIY], xiz = in.m[XIZ];
+    const R etx = in.m[ETX], ety = in.m[ETY], etz = in.m[ETZ];
+    const R ztx = in.m[ZTX], zty = in.m[ZTY], ztz = in.m[ZTZ];
+    R qx[NO], qy[NO], qz[NO];
+    R s1[3] = {0, 0, 0}, s2[3] = {0, 0, 0};
+    R lam2mu = 0, miu = 0, lambda = 0;
+    if constexpr (PART == 0) {
+        constexpr int XX = 0, YY = 1, ZZ = 2, XY = 3, XZ = 4, YZ = 5;
+        const R rho = in.med[0];
+        if (!HY || z >= a->zcon) {
+            qx[0] = (xix * Dx[XX] + xiy * Dx[XY] + xiz * Dx[XZ]) * rho;
+            qy[0] = (etx * Dy[XX] + ety * Dy[XY] + etz * Dy[XZ]) * rho;
+            qz[0] = (ztx * Dz[XX] + zty * Dz[XY] + ztz * Dz[XZ]) * rho;
+            qx[1] = (xix * Dx[XY] + xiy * Dx[YY] + xiz * Dx[YZ]) * rho;
+            qy[1] = (etx * Dy[XY] + ety * Dy[YY] + etz * Dy[YZ]) * rho;
+            qz[1] = (ztx * Dz[XY] + zty * Dz[YY] + ztz * Dz[YZ]) * rho;
+            qx[2] = (xix * Dx[XZ] + xiy * Dx[YZ] + xiz * Dx[ZZ]) * rho;
+            qy[2] = (etx * Dy[XZ] + ety * Dy[YZ] + etz * Dy[ZZ]) * rho;
+            qz[2] = (ztx * Dz[XZ] + zty * Dz[YZ] + ztz * Dz[ZZ]) * rho;
+        } else {
+            qx[0] = rho * xix * Dx[XX];
+            qy[0] = rho * ety * Dy[XY];
+            qz[0] = ztz * Dz[XZ] * rho;
+            qx[1] = rho * xix * Dx[XY];
+            qy[1] = rho * ety * Dy[YY];
+            qz[1] = ztz * Dz[YZ] * rho;
+            qx[2] = rho * xix * Dx[XZ];
+            qy[2] = rho * ety * Dy[YZ];
+            qz[2] = ztz * Dz[ZZ] * rho;
+        }
+    } else {
+        // velocity zeta-derivatives of the top three rows
+        if (top == 2) {
+            R cx[9], cy[9];
+#pragma unroll
+            for (int m = 0; m < 9; ++m) {
+                cx[m] = a->cov[m * a->cstr + cxy];
+                cy[m] = a->cov[(9 + m) * a->cstr + cxy];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                s1[c] = cx[3 * c] * Dx[0] + cx[3 * c + 1] * Dx[1] + cx[3 * c + 2] * Dx[2];
+                s2[c] = cy[3 * c] * Dy[0] + cy[3 * c + 1] * Dy[1] + cy[3 * c + 2] * Dy[2];
+                Dz[c] = s1[c] + cy[3 * c] * Dy[0] + cy[3 * c + 1] * Dy[1] + cy[3 * c + 2] * Dy[2];
+            }
+        } else if (top == 1) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) Dz[c] = SZ > 0 ? (w[c][2] - w[c][1]) / a->hr : (w[c][3] - w[c][2]) / a->hr;
+        } else if (top == 0) {
+            const double h = a->h;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                double s = SZ > 0 ? M24A0 * (double)w[c][1] + M24A1 * (double)w[c][2] + M24A2 * (double)w[c][3]
+                                  : M24A2 * (double)w[c][1] + M24A1 * (double)w[c][2] + M24A0 * (double)w[c][3];
+                Dz[c] = (R)(SZ > 0 ? s / h : s / (-h));
+            }
+        }
+        lam2mu = in.med[0];
+        miu = in.med[1];
+        lambda = lam2mu - (R)2 * miu;
+        if (!HY || z >= a->zcon) {
+            qx[0] = lam2mu * xix * Dx[0] + lambda * xiy * Dx[1] + lambda * xiz * Dx[2];
+            qy[0] = lam2mu * etx * Dy[0] + lambda * ety * Dy[1] + lambda * etz * Dy[2];
+            qz[0] = lam2mu * ztx * Dz[0] + lambda * zty * Dz[1] + lambda * ztz * Dz[2];
+            qx[1] = lambda * xix * Dx[0] + lam2mu * xiy * Dx[1] + lambda * xiz * Dx[2];
+            qy[1] = lambda * etx * Dy[0] + lam2mu * ety * Dy[1] + lambda * etz * Dy[2];
+            qz[1] = lambda * ztx * Dz[0] + lam2mu * zty * Dz[1] + lambda * ztz * Dz[2];
+            qx[2] = lambda * xix * Dx[0] + lambda * xiy * Dx[1] + lam2mu * xiz * Dx[2];
+            qy[2] = lambda * etx * Dy[0] + lambda * ety * Dy[1] + lam2mu * etz * Dy[2];
+            qz[2] = lambda * ztx * Dz[0] + lambda * zty * Dz[1] + lam2mu * ztz * Dz[2];
+            qx[3] = (xiy * Dx[0] + xix * Dx[1]) * miu;
+            qy[3] = (ety * Dy[0] + etx * Dy[1]) * miu;
+            qz[3] = (zty * Dz[0] + ztx * Dz[1]) * miu;
+            qx[4] = (xiz * Dx[0] + xix * Dx[2]) * miu;
+            qy[4] = (etz * Dy[0] + etx * Dy[2]) * miu;
+            qz[4] = (ztz * Dz[0] + ztx * Dz[2]) * miu;
+            qx[5] = (xiz * Dx[1] + xiy * Dx[2]) * miu;
+            qy[5] = (etz * Dy[1] + ety * Dy[2]) * miu;
+            qz[5] = (ztz * Dz[1] + zty * Dz[2]) * miu;
+        } else {
+            qx[0] = lam2mu * xix * Dx[0];
+            qy[0] = lambda * ety * Dy[1];
+            qz[0] = lambda * ztz * Dz[2];
+            qx[1] = lambda * xix * Dx[0];
+            qy[1] = lam2mu * ety * Dy[1];
+            qz[1] = lambda * ztz * Dz[2];
+            qx[2] = lambda * xix * Dx[0];
+            qy[2] = lambda * ety * Dy[1];
+            qz[2] = lam2mu * ztz * Dz[2];
+            qx[3] = miu * xix * Dx[1];
+            qy[3] = miu * ety * Dy[0];
+            qz[3] = (R)0;
+            qx[4] = miu * xix * Dx[2];
+            qy[4] = (R)0;
+            qz[4] = ztz * Dz[0] * miu;
+            qx[5] = (R)0;
+            qy[5] = miu * ety * Dy[2];
+            qz[5] = ztz * Dz[1] * miu;
+        }
+    }
+    const R Bz = pmz[g.nk + z];
+    // x/1 is x: an axis whose CFS factor is 1 skips its divisions
+    R d[NO];
+#pragma unroll
+    for (int c = 0; c < NO; ++c) hv[c] = qx[c];
+    const R Bx = k.Bx, By = k.By;
+    if (Bx != (R)1) {
+#pragma unroll
+        for (int c = 0; c < NO; ++c) hv[c] = qx[c] / Bx;
+    }
+#pragma unroll
+    for (int c = 0; c < NO; ++c) d[c] = qy[c];
+    if (By != (R)1) {
+#pragma unroll
+        for (int c = 0; c < NO; ++c) d[c] = qy[c] / By;
+    }
+#pragma unroll
+    for (int c = 0; c < NO; ++c) {
+        hv[c] = hv[c] + d[c];
+        d[c] = qz[c];
+    }
+    if (Bz != (R)1) {
+#pragma unroll
+        for (int c = 0; c < NO; ++c) d[c] = qz[c] / Bz;
+    }
+#pragma unroll
+    for (int c = 0; c < NO; ++c) hv[c] = hv[c] + d[c];
+
+    const unsigned tcell = (unsigned)(top > 0 ? top : 0) * (unsigned)(g.nj * g.nxp) + cxy;
+    if (k.inx) {
+        const R APDx = k.APDx, DBx = k.DBx;
+        const int ix = x < a->nabs[0] ? x : x - (g.ni - a->nabs[1]) + a->nabs[0];
+        const long aidx = ((long)z * g.nj + y) * a->npml[0] + ix;
+        HalfAux<R, PART> v;
+        load_half_aux<R, ST, PART>(a, 0, aidx, v);
+        R ha[NO];
+        aux_rates<R, PART>(qx, v, Bx, DBx, APDx, hv, ha);
+        if constexpr (PART == 0) {
+            if (top >= 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) ha[c] = a->timg[(3 + c) * a->tstr + tcell];
+            }
+        } else {
+            if (top == 2) surface_stress<R>(DBx * Bx, lam2mu, lambda, miu, in.m, s1[0], s1[1], s1[2], ha);
+        }
+        store_half_aux<R, ST, PART>(a, 0, aidx, v, ha);
+    }
+    if (k.iny) {
+        const R APDy = k.APDy, DBy = k.DBy;
+        const int iy = y < a->nabs[2] ? y : y - (g.nj - a->nabs[3]) + a->nabs[2];
+        const long aidx = ((long)z * a->npml[1] + iy) * g.nxp + x;
+        HalfAux<R, PART> v;
+        load_half_aux<R, ST, PART>(a, 1, aidx, v);
+        R ha[NO];
+        aux_rates<R, PART>(qy, v, By, DBy, APDy, hv, ha);
+        if constexpr (PART == 0) {
+            if (top >= 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) ha[c] = a->timg[(6 + c) * a->tstr + tcell];
+            }
+        } else {
+            if (top == 2) surface_stress<R>(DBy * By, lam2mu, lambda, miu, in.m, s2[0], s2[1], s2[2], ha);
+        }
+        store_half_aux<R, ST, PART>(a, 1, aidx, v, ha);
+    }
+    if (z < a->nabs[4] || z >= g.nk - a->nabs[5]) {
+        const int iz = z < a->nabs[4] ? z : z - (g.nk - a->nabs[5]) + a->nabs[4];
+        const long aidx = ((long)iz * g.nj + y) * g.nxp + x;
+        const R APDz = pmz[z], DBz = pmz[2 * g.nk + z];
+        HalfAux<R, PART> v;
+        load_half_aux<R, ST, PART>(a, 2, aidx, v);
+        R ha[NO];
+        aux_rates<R, PART>(qz, v, Bz, DBz, APDz, hv, ha);
+        store_half_aux<R, ST, PART>(a, 2, aidx, v, ha);
+    }
+    if (PART == 0 && top >= 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) hv[c] = a->timg[c * a->tstr + tcell];
+    }
+    if (e >= 0) {
+        const int col = y * g.ni + x;
+        int4 en = a->sent[e];
+        while (en.w == col && en.x == z) {
+            const R *cf = a->scoef + (long)e * 8;
+            if (PART == 0 && en.y == 0) {
+                const R stf = a->fstf[(long)en.z * a->nstf_f + tindex];
+                const R A = cf[0];
+                hv[0] += stf * cf[1] * A;
+                hv[1] += stf * cf[2] * A;
+                hv[2] += stf * cf[3] * A;
+            } else if (PART == 1 && en.y == 1) {
+                const R stf = a->mstf[(long)en.z * a->nstf_m + tindex];
+                R A = (R)1;
+                A = stf * A / cf[0];
+#pragma unroll
+                for (int c = 0; c < NO; ++c) hv[c] -= cf[1 + c] * A;
+            } else if (PART == 1 && en.y == 2) {
+                const R *fv = a->rstf + (long)en.z * 6 * a->nstf_r + tindex;
+                const R A = cf[0];
+#pragma unroll
+                for (int c = 0; c < NO; ++c) hv[c] -= fv[(long)c * a->nstf_r] * A;
+            }
+            en = a->sent[++e];
+        }
+    }
+}
+
+// Wavefronts per SIMD in FP32: 4 with constant horizontal metrics; all nine
+// metrics spill 5-19 registers at 4 (149x131x97: 155 us against 149 at 3).
+#ifndef CGFD_HALF_WAVES
+#define CGFD_HALF_WAVES ((HM & 1) ? 4 : 3)
+#endif
+#define CGFD_HALF_ATTR __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? CGFD_HALF_WAVES : 2, 8)))
+
+constexpr int HALF_TY = 4; // wavefronts per workgroup
+
+template <typename R, int SX, int SZ, int ST, int HM, int TW, int PART, typename AP>
+__device__ __forceinline__ void half_sweep(const AP a0, int L, R *ldsbuf)
+{
+    constexpr int NIN = Half<PART>::NIN, I0 = Half<PART>::I0, NO = Half<PART>::NO, O0 = Half<PART>::O0;
+    constexpr int TY = HALF_TY, HALVES = 64 / TW, TR = TY * HALVES;
+    constexpr int HX = TW + 4, HY = TR + 4;
+    constexpr int O = SX > 0 ? 1 : 3;
+    constexpr int ZOFF = SZ > 0 ? -1 : -3;
+    constexpr int CI = SZ > 0 ? 1 : 3;
+    constexpr int D = ZOFF + 4;
+    typedef R Tile[NIN][HY][HX];
+    Tile *lds = (Tile *)ldsbuf; // two plane tiles
+
+    const int tinc = ST == 0 ? 0 : (ST < 3 ? 1 : 2);
+    const int tindex = 2 * *a0->step + tinc;
+    const Geom g = geom_of(a0);
+    // threadIdx.y is the wavefront: uniform, so rows of 64-column tiles live in
+    // scalar registers
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int part = TW == 64 ? 0 : lane / TW;
+    const int tx = TW == 64 ? lane : lane % TW, ty = wv * HALVES + part;
+    const int ntx = (g.ni + TW - 1) / TW, nty = (g.nj + TR - 1) / TR;
+    const int bx = L % ntx, by = (L / ntx) % nty, bz = L / (ntx * nty);
+    const int x0 = bx * TW, y0 = by * TR;
+    const int x = x0 + tx, y = y0 + ty;
+    const bool active = x < g.ni && y < g.nj;
+    const int z0 = bz * a0->zlen;
+    const int z1 = min(g.nk, z0 + a0->zlen);
+    if (z0 >= z1) return; // uniform over the workgroup
+
+    const long fs0 = g.fs;
+    const double h = a0->h, rh = a0->rh;
+    const unsigned esz = sizeof(R);
+    const unsigned plb = (unsigned)(g.plane * esz);
+    const int yc = min(y, g.nyp - 1);
+    // Halo slots of this lane.  Rows: wavefront hk stages halo row hk; with two
+    // tile rows per wavefront each part of it takes half the components.
+    // Columns: the 4*TR slots of a component go to one part of a wavefront;
+    // slots past the last component reload it and drop the value, so every
+    // lane issues the same loads.
+    const int hk = wv;
+    const int hrow = SX > 0 ? (hk == 0 ? 0 : TR + hk) : (hk < 3 ? hk : TR + 3);
+    const int hy = y0 - O + hrow, hxx = x0 + tx;
+    const bool hv1 = hy >= -3 && hy < g.nyp;
+    constexpr int NR = (NIN + HALVES - 1) / HALVES;
+#define CGFD_HALF_FIELD(j) (TW == 64 ? (j) : min(part * NR + (j), NIN - 1))
+    constexpr int NH = (NIN + TY * HALVES - 1) / (TY * HALVES);
+    const bool xlane = tx < 4 * TR;
+    const int hc2k = tx / TR, hr2 = tx % TR;
+    const int hcol = SX > 0 ? (hc2k == 0 ? 0 : TW + hc2k) : (hc2k < 3 ? hc2k : TW + 3);
+    const int hx2 = x0 - O + hcol, hy2 = y0 + hr2;
+    const bool hv2 = xlane && hx2 >= -3 && hx2 < g.nxp && hy2 < g.nyp;
+    auto hfield = [&](int j) { return min(hk + TY * (HALVES * j + part), NIN - 1); };
+    auto hkeep = [&](int j) { return xlane && hk + TY * (HALVES * j + part) < NIN; };
+    const int rel_c = (yc * g.nxp + x) * (int)esz;
+    const unsigned base0 = (unsigned)(g.base * esz);
+    auto pbase = [&](int zz) { return base0 + (unsigned)zz * plb; };
+    // halo slots outside the padded field read offset 0, a guard cell that is
+    // always zero
+    unsigned off1 = hv1 ? pbase(z0) + (hy * g.nxp + hxx) * (int)esz : 0, inc1 = hv1 ? plb : 0;
+    unsigned off2 = hv2 ? pbase(z0) + (hy2 * g.nxp + hx2) * (int)esz : 0, inc2 = hv2 ? plb : 0;
+
+    HalfCol<R> k;
+    {
+        const int xs = active ? x : 0, ys = active ? y : 0;
+        k.inx = xs < a0->nabs[0] || xs >= g.ni - a0->nabs[1];
+        k.iny = ys < a0->nabs[2] || ys >= g.nj - a0->nabs[3];
+        const R *pmx = a0->pml, *pmy = pmx + 3 * g.ni;
+        k.APDx = pmx[xs];
+        k.Bx = pmx[g.ni + xs];
+        k.DBx = pmx[2 * g.ni + xs];
+        k.APDy = pmy[ys];
+        k.By = pmy[g.nj + ys];
+        k.DBy = pmy[2 * g.nj + ys];
+    }
+    int e = active ? first_source(a0, y * g.ni + x, z0) : -1;
+
+    const R *win0 = a0->win + I0 * fs0;
+    R w[NIN][5];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < NIN; ++c) w[c][j] = ldg(win0 + c * fs0, pbase(z0 + ZOFF + j) + rel_c);
+    R lead[NIN], h1[NR], h2[NH];
+#pragma unroll
+    for (int c = 0; c < NIN; ++c) lead[c] = ldg(win0 + c * fs0, pbase(z0 + D) + rel_c);
+#pragma unroll
+    for (int j = 0; j < NR; ++j) h1[j] = ldg(win0 + CGFD_HALF_FIELD(j) * fs0, off1);
+#pragma unroll
+    for (int j = 0; j < NH; ++j) h2[j] = ldg(win0 + hfield(j) * fs0, off2);
+
+    for (int z = z0; z < z1; ++z) {
+        // laundered once per plane, so that the field addresses derived from
+        // it are rebuilt on the scalar unit instead of held (and spilled)
+        long fs = g.fs;
+        asm volatile("" : "+s"(fs));
+        AP al = a0;
+        asm volatile("" : "+s"(al));
+        const unsigned pbz = pbase(z) + rel_c;
+        HalfIn<R, PART> cin;
+        load_half<R, ST, (HM & 1), PART>(al, pbz, fs, cin);
+        // Two plane tiles in turn: a wavefront writes tile z while others
+        // still read tile z-1; the tile of z-2 was last read before every
+        // wavefront reached the barrier of z-1.
+        Tile &T = lds[z & 1];
+#pragma unroll
+        for (int c = 0; c < NIN; ++c) {
+            T[c][O + ty][O + tx] = w[c][CI];
+            w[c][4] = lead[c];
+        }
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+            if (TW == 64 || part * NR + j < NIN) T[CGFD_HALF_FIELD(j)][hrow][O + tx] = h1[j];
+#pragma unroll
+        for (int j = 0; j < NH; ++j)
+            if (hkeep(j)) T[hfield(j)][O + hr2][hcol] = h2[j];
+        __syncthreads();
+        const R *win = al->win + I0 * fs;
+        off1 += inc1;
+        off2 += inc2;
+#pragma unroll
+        for (int c = 0; c < NIN; ++c) lead[c] = ldg(win + c * fs, pbase(z + 1 + D) + rel_c);
+#pragma unroll
+        for (int j = 0; j < NR; ++j) h1[j] = ldg(win + CGFD_HALF_FIELD(j) * fs, off1);
+#pragma unroll
+        for (int j = 0; j < NH; ++j) h2[j] = ldg(win + hfield(j) * fs, off2);
+        R hv[NO];
+#pragma unroll
+        for (int c = 0; c < NO; ++c) hv[c] = (R)0;
+        if (active) {
+            R Dx[NIN], Dy[NIN], Dz[NIN];
+#pragma unroll
+            for (int c = 0; c < NIN; ++c) {
+                const R ctr = w[c][CI];
+                const R *rx = &T[c][O + ty][tx];
+                const R *ry = &T[c][ty][O + tx];
+                if (SX > 0) {
+                    Dx[c] = dfd<R, 1>(rx[0], ctr, rx[2], rx[3], rx[4], h, rh);
+                    Dy[c] = dfd<R, 1>(ry[0], ctr, ry[2 * HX], ry[3 * HX], ry[4 * HX], h, rh);
+                } else {
+                    Dx[c] = dfd<R, -1>(rx[0], rx[1], rx[2], ctr, rx[4], h, rh);
+                    Dy[c] = dfd<R, -1>(ry[0], ry[HX], ry[2 * HX], ctr, ry[4 * HX], h, rh);
+                }
+                Dz[c] = dfd<R, SZ>(w[c][0], w[c][1], w[c][2], w[c][3], w[c][4], h, rh);
+            }
+            half_rates<R, SX, SZ, ST, (HM >> 1), PART>(al, k, cin, Dx, Dy, Dz, w, x, y, z, e, tindex, hv);
+        }
+        const unsigned fb = (unsigned)(fs * (long)sizeof(R));
+#pragma unroll
+        for (int c = 0; c < NO; ++c) {
+            R *wo = al->wout + (O0 + c) * fs, *to = al->tw + (O0 + c) * fs;
+            if (ST == 0) {
+                stg_keep(wo, pbz, cin.fw[c] + al->alpha * hv[c], active, fb);
+                stg_keep(to, pbz, cin.fw[c] + al->beta * hv[c], active, fb);
+            } else if (ST < 3) {
+                stg_keep(wo, pbz, cin.fw[c] + al->alpha * hv[c], active, fb);
+                stg_keep(to, pbz, cin.tw[c] + al->beta * hv[c], active, fb);
+            } else {
+                const R wn = cin.tw[c] + al->beta * hv[c];
+                stg_keep(wo, pbz, wn, active, fb);
+                if (PART == 0 && active && z == g.nk - 1 && al->pgv) {
+                    R *pv = al->pgv + c * al->cstr + (unsigned)(y * g.nxp + x);
+                    *pv = rmax(rabs(wn), rabs(*pv));
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NIN; ++c) {
+            w[c][0] = w[c][1];
+            w[c][1] = w[c][2];
+            w[c][2] = w[c][3];
+            w[c][3] = w[c][4];
+        }
+    }
+#undef CGFD_HALF_FIELD
+}
+
+// One launch covers every grid, tile, chunk and half.  The argument block lies
+// in device memory and is read through the constant address space, field by
+// field where it is used.  A batched launch (nctx > 1) covers several grids:
+// grid c owns the tiles starts[c] .. starts[c+1]-1 and its block lies c *
+// kCtxArgBytes after pa; with nctx = -n the n grids are identical and on one
+// medium.  Workgroups are dealt round-robin to the 8 XCDs: the two halves of a
+// tile follow each other on one XCD, whose L2 then holds the metrics both
+// read, and so do the copies of a tile of grids that share a medium.  Each XCD
+// gets a uniform sample of the domain, so none ends late with the absorbing
+// layers.
+template <typename R, int SX, int SZ, int ST, int HM, int TW>
+__global__ void __launch_bounds__(64 * HALF_TY) CGFD_HALF_ATTR
+stage_half_kernel(const StageArgs<R> *pa, const int *starts, int nctx)
+{
     typedef const __attribute__((address_space(4))) StageArgs<R> *AP;
     typedef const __attribute__((address_space(4))) int *SP;
-    int ctx = 0, nb = gridDim.x, id = blockIdx.x;
+    constexpr int TR = HALF_TY * (64 / TW);
+    __shared__ R lds[2 * 6 * (TR + 4) * (TW + 4)];
+    int ctx = 0;
+    const int W = gridDim.x >> 1, b = blockIdx.x; // W tiles (times chunks) in the launch
+    int part, id;
+    if (b < (W & ~7) * 2) { // 8 tiles, one per XCD, then their other halves
+        part = (b >> 3) & 1;
+        id = (b >> 4) * 8 + (b & 7);
+    } else {
+        const int r = b - (W & ~7) * 2;
+        part = r & 1;
+        id = (W & ~7) + (r >> 1);
+    }
     if (nctx < 0) {
-        // n identical grids on one medium: workgroups are dealt round-robin
-        // to the 8 XCDs, and the n copies of one tile follow each other on
-        // one XCD, which reads the metric and media lines they share from
-        // its L2.  Tiles past the last multiple of 8 run grid after grid.
+        // the n copies of each tile one after another on one XCD; tiles past
+        // the last multiple of 8 run grid after grid
         const int n = -nctx;
-        nb = gridDim.x / n;
+        const int nb = W / n;
         const int M = (nb >> 3) * 8 * n;
         if (id < M) {
             const int k = id >> 3;
@@ -731,235 +1263,13 @@ stage_lds_kernel(const StageArgs<R> *pa, const int *starts, int nctx, int tinc)
             else hi = mid - 1;
         }
         ctx = lo;
-        nb = st[lo + 1] - st[lo];
         id -= st[lo];
     }
     const AP a0 = (AP)((const char *)pa + (long)ctx * kCtxArgBytes);
-    const int tindex = 2 * *a0->step + tinc;
-    // A workgroup of TY wavefronts owns a tile of TW columns x TR rows: with
-    // TW = 64 a wavefront is one tile row, with TW = 32 it holds two (rows
-    // whose length leaves a short last 64-column tile waste fewer lanes).
-    static_assert(TW == 64 || TW == 32, "tile width");
-    constexpr int TY = lds_ty<R>(), HALVES = 64 / TW, TR = TY * HALVES;
-    constexpr int HX = TW + 4, HY = TR + 4;
-    constexpr int O = SX > 0 ? 1 : 3; // halo cells below the tile in x and in y
-    constexpr int ZOFF = SZ > 0 ? -1 : -3;
-    constexpr int CI = SZ > 0 ? 1 : 3;
-    // The window lead of plane z is plane z+D.  With the halo ring, the halo
-    // rows and columns of a plane are fetched in the same iteration as its
-    // lead, i.e. when the neighbouring tiles fetch those same lines as their
-    // own lead (so they are still in L2), and wait in an LDS ring of D+1
-    // plane tiles until the plane becomes the centre.
-    constexpr int D = ZOFF + 4;
-    constexpr int HD = CGFD_HALO_RING ? D : 0; // halo prefetch distance
-    constexpr int NSLOT = HD + 1;              // 4, 2 or 1 plane tiles
-    typedef R LT;                              // type of the plane tiles
-    __shared__ LT lds[NSLOT][NF][HY][HX];
-    auto slot = [](int p) { return p & (NSLOT - 1); };
-
-    const AP a = a0;
-    const Geom g = geom_of(a);
-    const int lane = threadIdx.x, wv = threadIdx.y;
-    // which tile row of its wavefront the lane is in (blockDim.x is 64)
-    const int part = TW == 64 ? 0 : lane / TW;
-    const int tx = TW == 64 ? lane : lane % TW, ty = wv * HALVES + part;
-
-    // Tile numbering.  Workgroups are dealt round-robin to the 8 XCDs, so
-    // the identity map (default) gives every XCD a uniform sample of the
-    // domain (the same share of PML, surface and source work) and keeps the
-    // running workgroups inside one z chunk.  Map 0 gives each XCD a
-    // contiguous run of tiles (neighbours share its L2, but the XCDs holding
-    // the bottom PML planes finish last); map 4 does that within groups of
-    // 8*CGFD_TILE_GROUP consecutive tiles.  Both cut the L2 fetch traffic by
-    // ~8 % on the 600x600x300 model yet run slower than the identity map.
-    const int ntx = (g.ni + TW - 1) / TW, nty = (g.nj + TR - 1) / TR;
-#ifndef CGFD_TILE_MAP
-#define CGFD_TILE_MAP 1
-#endif
-#if CGFD_TILE_MAP == 1
-    const int L = id;
-#elif CGFD_TILE_MAP == 5
-    // whole rows of x tiles on one XCD (x neighbours share its L2), rows
-    // dealt round-robin to the XCDs; the rows past the last multiple of 8
-    // keep the identity map
-    const int nrow = nb / ntx, M = (nrow / 8) * 8 * ntx;
-    int L = id;
-    if (id < M) {
-        const int k = id / 8;
-        L = ((k / ntx) * 8 + id % 8) * ntx + k % ntx;
-    }
-#elif CGFD_TILE_MAP == 4
-    // groups of 8*S consecutive tiles (about what the chip runs at once);
-    // inside a group each XCD takes a contiguous run
-#ifndef CGFD_TILE_GROUP
-#define CGFD_TILE_GROUP 64
-#endif
-    constexpr int G = 8 * CGFD_TILE_GROUP;
-    const int gbase = id / G * G, rem = min(G, nb - gbase), wi = id - gbase;
-    const int q = rem / 8, r = rem % 8, xcd = wi % 8;
-    const int L = gbase + xcd * q + min(xcd, r) + wi / 8;
-#else
-    const int q = nb / 8, r = nb % 8, xcd = id % 8;
-    const int L = xcd * q + min(xcd, r) + id / 8;
-#endif
-    const int bx = L % ntx, by = (L / ntx) % nty, bz = L / (ntx * nty);
-    const int x0 = bx * TW, y0 = by * TR;
-    const int x = x0 + tx, y = y0 + ty;
-    const bool active = x < g.ni && y < g.nj;
-    const int z0 = bz * a->zlen;
-    const int z1 = min(g.nk, z0 + a->zlen);
-    if (z0 >= z1) return; // uniform over the workgroup
-
-    const long fs0 = g.fs;
-    const double h = a->h, rh = a->rh;
-    const unsigned esz = sizeof(R);
-    const unsigned plb = (unsigned)(g.plane * esz); // bytes per plane
-
-    // Addresses.  x < ntx*TW <= nxp always; rows past the last guard row
-    // (y >= nyp, only in a ragged last tile) are clamped onto it (a zero row),
-    // so every load stays inside its own plane.
-    const int yc = min(y, g.nyp - 1);
-    // Halo slots of this lane.  Halo rows: wavefront hk (the first 4) stages
-    // halo row hk (TW columns); with two tile rows per wavefront its lanes of
-    // part 0 take fields 0-4 of that row and those of part 1 fields 5-8, so
-    // a lane stages NR fields.  Halo columns: the 4*TR slots of one field
-    // (4 columns x TR rows) go to lanes q = lane % TW < 4*TR of one part;
-    // wavefront hk, part p stages fields hk + TY*(HALVES*j + p), j < NH.
-    // Slots past the last field reload field 8 and discard it, so every
-    // lane issues the same loads.
-    const int hk = wv;
-    const int hrow = SX > 0 ? (hk == 0 ? 0 : TR + hk) : (hk < 3 ? hk : TR + 3);
-    const int hy = y0 - O + hrow, hxx = x0 + tx;
-    const bool hv1 = hk < 4 && hy >= -3 && hy < g.nyp;
-    constexpr int NR = (NF + HALVES - 1) / HALVES;
-    // field of halo-row slot j; a plain expression rather than a lambda,
-    // whose call inside a field address kept the 64-column kernel's field
-    // bases out of scalar registers (36 more 64-bit vector adds)
-#define CGFD_HRFIELD(j) (TW == 64 ? (j) : min(part * NR + (j), NF - 1))
-    auto hrkeep = [&](int j) { return hk < 4 && part * NR + j < NF; };
-    constexpr int NH = (NF + TY * HALVES - 1) / (TY * HALVES);
-    const bool xlane = tx < 4 * TR;
-    const int hc2k = tx / TR, hr2 = tx % TR;
-    const int hcol = SX > 0 ? (hc2k == 0 ? 0 : TW + hc2k) : (hc2k < 3 ? hc2k : TW + 3);
-    const int hx2 = x0 - O + hcol, hy2 = y0 + hr2;
-    const bool hv2 = xlane && hx2 >= -3 && hx2 < g.nxp && hy2 < g.nyp;
-    auto hfield = [&](int j) { return min(hk + TY * (HALVES * j + part), NF - 1); };
-    auto hkeep = [&](int j) { return xlane && hk + TY * (HALVES * j + part) < NF; };
-    // byte offsets inside plane 0 (may be negative: added to a plane base);
-    // invalid halo slots fall back to the lane's own cell
-    const int rel_c = (yc * g.nxp + x) * (int)esz;
-    const int rel_1 = hv1 ? (hy * g.nxp + hxx) * (int)esz : rel_c;
-    const int rel_2 = hv2 ? (hy2 * g.nxp + hx2) * (int)esz : rel_c;
-    const unsigned base0 = (unsigned)(g.base * esz);
-    auto pbase = [&](int zz) { return base0 + (unsigned)zz * plb; };
-
-    const Column<R> k = column_of<R>(a, active ? x : 0, active ? y : 0);
-    int e = active ? first_source(a, k.col, z0) : -1;
-
-    R w[NF][5];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int c = 0; c < NF; ++c) w[c][j] = ldg(a->win + c * fs0, pbase(z0 + ZOFF + j) + rel_c);
-
-    // halos of the planes z0 .. z0+HD-1 go straight into their ring tiles
-    for (int p = z0; p < z0 + HD; ++p) {
-#pragma unroll
-        for (int j = 0; j < NR; ++j) {
-            const R v1 = ldg(a->win + CGFD_HRFIELD(j) * fs0, pbase(p) + rel_1);
-            if (hrkeep(j)) lds[slot(p)][CGFD_HRFIELD(j)][hrow][O + tx] = (LT)(hv1 ? v1 : (R)0);
-        }
-#pragma unroll
-        for (int j = 0; j < NH; ++j) {
-            const R v2 = ldg(a->win + hfield(j) * fs0, pbase(p) + rel_2);
-            if (hkeep(j)) lds[slot(p)][hfield(j)][O + hr2][hcol] = (LT)(hv2 ? v2 : (R)0);
-        }
-    }
-
-    R lead[NF], h1[NR], h2[NH];
-#pragma unroll
-    for (int c = 0; c < NF; ++c) {
-        lead[c] = ldg(a->win + c * fs0, pbase(z0 + D) + rel_c);
-        if (c < NR) h1[c] = ldg(a->win + CGFD_HRFIELD(c) * fs0, pbase(z0 + HD) + rel_1);
-    }
-#pragma unroll
-    for (int j = 0; j < NH; ++j) h2[j] = ldg(a->win + hfield(j) * fs0, pbase(z0 + HD) + rel_2);
-
-    for (int z = z0; z < z1; ++z) {
-        // The field stride is laundered through an empty asm once per plane,
-        // so the ~40 per-field base addresses derived from it are rebuilt on
-        // the scalar unit each plane instead of being held (and spilled)
-        // across the whole sweep.
-        long fs = g.fs;
-        asm volatile("" : "+s"(fs));
-        AP al = a0;
-        asm volatile("" : "+s"(al));
-        // Every lane loads its cell inputs and stores its results without a
-        // branch: a lane outside the grid addresses its own zero guard cell
-        // (x in [ni, nxp) or a clamped guard row) and reads zeros; its stores
-        // are dropped (rk_store).  With no skippable memory operation between
-        // them, the compiler's wait counts let this plane's cell loads stay in
-        // flight while the previous plane's prefetch is consumed.
-        const unsigned pbz = pbase(z) + rel_c;
-        CellIn<R> cin;
-        load_cell<R, ST, (HM & 1)>(al, pbz, fs, cin);
-        __syncthreads(); // the previous plane's LDS reads are done (its tile is slot(z+HD) now)
-        const int sc = slot(z), sh = slot(z + HD);
-#pragma unroll
-        for (int c = 0; c < NF; ++c) {
-            lds[sc][c][O + ty][O + tx] = (LT)w[c][CI];
-            if (c < NR && hrkeep(c)) lds[sh][CGFD_HRFIELD(c)][hrow][O + tx] = (LT)(hv1 ? h1[c] : (R)0);
-            w[c][4] = lead[c];
-        }
-#pragma unroll
-        for (int j = 0; j < NH; ++j)
-            if (hkeep(j)) lds[sh][hfield(j)][O + hr2][hcol] = (LT)(hv2 ? h2[j] : (R)0);
-        __syncthreads();
-        // next plane's lead (plane z+1+D <= nk+3) and halo (plane z+1+HD <=
-        // nk+3) lie inside the 4 zero planes above the grid
-#pragma unroll
-        for (int c = 0; c < NF; ++c) {
-            lead[c] = ldg(al->win + c * fs, pbase(z + 1 + D) + rel_c);
-            if (c < NR) h1[c] = ldg(al->win + CGFD_HRFIELD(c) * fs, pbase(z + 1 + HD) + rel_1);
-        }
-#pragma unroll
-        for (int j = 0; j < NH; ++j) h2[j] = ldg(al->win + hfield(j) * fs, pbase(z + 1 + HD) + rel_2);
-        R hv[NF];
-#pragma unroll
-        for (int c = 0; c < NF; ++c) hv[c] = (R)0;
-        if (active) {
-            R Dx[NF], Dy[NF], Dz[NF];
-#pragma unroll
-            for (int c = 0; c < NF; ++c) {
-                const LT ctr = (LT)w[c][CI];
-                const LT *rx = &lds[sc][c][O + ty][tx]; // taps x-O .. x-O+4
-                const LT *ry = &lds[sc][c][ty][O + tx]; // taps y-O .. y-O+4
-                if (SX > 0) {
-                    Dx[c] = dfd<R, 1>(rx[0], ctr, rx[2], rx[3], rx[4], h, rh);
-                    Dy[c] = dfd<R, 1>(ry[0], ctr, ry[2 * HX], ry[3 * HX], ry[4 * HX], h, rh);
-                } else {
-                    Dx[c] = dfd<R, -1>(rx[0], rx[1], rx[2], ctr, rx[4], h, rh);
-                    Dy[c] = dfd<R, -1>(ry[0], ry[HX], ry[2 * HX], ctr, ry[4 * HX], h, rh);
-                }
-                Dz[c] = dfd<R, SZ>(w[c][0], w[c][1], w[c][2], w[c][3], w[c][4], h, rh);
-            }
-            cell_rates<R, SX, SZ, ST, (HM >> 1)>(al, k, cin, Dx, Dy, Dz, w, x, y, z, e, tindex, hv);
-        }
-        // lanes outside the grid: their buffer stores are dropped (FP32), or
-        // their zero inputs and zero rates store zeros (FP64)
-        rk_store<R, SZ, ST>(al, cin, w, hv, pbz, fs, active);
-        if (active) pgv_update<R, ST>(al, k, cin, hv, z - (g.nk - 3));
-#pragma unroll
-        for (int c = 0; c < NF; ++c) {
-            w[c][0] = w[c][1];
-            w[c][1] = w[c][2];
-            w[c][2] = w[c][3];
-            w[c][3] = w[c][4];
-        }
-    }
+    if (part == 0) half_sweep<R, SX, SZ, ST, HM, TW, 0>(a0, id, lds);
+    else half_sweep<R, SX, SZ, ST, HM, TW, 1>(a0, id, lds);
 }
 
-#undef CGFD_HRFIELD
 
 // ---------------------------------------------------------------------------
 // Variant "split": each stage as two kernels, one per half of the system.
@@ -1749,24 +2059,22 @@ __global__ void snap_kernel(const R *fw, long fs, const long *lin, int npts, int
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// The LDS kernel at the tile width a.tile (32 or 64 columns; FP64 always 64).
+// The half-system kernel at the tile width a.tile (32 or 64 columns; FP64 always 64).
 template <typename R, int SX, int SZ, int ST, int HM>
-static void launch_lds(const StageArgs<R> &a, const StageArgs<R> *pa, const int *starts, int nctx, int nblocks,
-                       int tinc, int zchunks, hipStream_t s)
+static void launch_half(const StageArgs<R> &a, const StageArgs<R> *pa, const int *starts, int nctx, int nblocks,
+                        int zchunks, hipStream_t s)
 {
-    constexpr int ty = lds_ty<R>();
-    const dim3 block(64, ty);
+    const int tw = sizeof(R) == 4 ? a.tile : 64, tr = stage_tile_rows(sizeof(R) == 8, tw);
+    const int ntx = (a.g.ni + tw - 1) / tw, nty = (a.g.nj + tr - 1) / tr;
+    // two workgroups per tile, one per half of the system
+    const dim3 grid(2u * (unsigned)(nblocks > 0 ? nblocks : ntx * nty * zchunks)), block(64, HALF_TY);
     if constexpr (sizeof(R) == 4) {
-        if (a.tile == 32) {
-            const int ntx = (a.g.ni + 31) / 32, nty = (a.g.nj + 2 * ty - 1) / (2 * ty);
-            const dim3 grid((unsigned)(nblocks > 0 ? nblocks : ntx * nty * zchunks));
-            stage_lds_kernel<R, SX, SZ, ST, HM, 32><<<grid, block, 0, s>>>(pa, starts, nctx, tinc);
+        if (tw == 32) {
+            stage_half_kernel<R, SX, SZ, ST, HM, 32><<<grid, block, 0, s>>>(pa, starts, nctx);
             return;
         }
     }
-    const int ntx = (a.g.ni + 63) / 64, nty = (a.g.nj + ty - 1) / ty;
-    const dim3 grid((unsigned)(nblocks > 0 ? nblocks : ntx * nty * zchunks));
-    stage_lds_kernel<R, SX, SZ, ST, HM, 64><<<grid, block, 0, s>>>(pa, starts, nctx, tinc);
+    stage_half_kernel<R, SX, SZ, ST, HM, 64><<<grid, block, 0, s>>>(pa, starts, nctx);
 }
 
 template <typename R, int SX, int SZ, int ST>
@@ -1777,10 +2085,10 @@ static void launch_stage_one(int variant, const StageArgs<R> &a, const StageArgs
         // mode bit 0: constant horizontal metrics; bit 1: a hybrid grid's
         // Cartesian planes
         switch ((a.hmet ? 1 : 0) | (a.zcon > 0 ? 2 : 0)) {
-        case 0: launch_lds<R, SX, SZ, ST, 0>(a, pa, starts, nctx, nblocks, tinc, zchunks, s); break;
-        case 1: launch_lds<R, SX, SZ, ST, 1>(a, pa, starts, nctx, nblocks, tinc, zchunks, s); break;
-        case 2: launch_lds<R, SX, SZ, ST, 2>(a, pa, starts, nctx, nblocks, tinc, zchunks, s); break;
-        default: launch_lds<R, SX, SZ, ST, 3>(a, pa, starts, nctx, nblocks, tinc, zchunks, s); break;
+        case 0: launch_half<R, SX, SZ, ST, 0>(a, pa, starts, nctx, nblocks, zchunks, s); break;
+        case 1: launch_half<R, SX, SZ, ST, 1>(a, pa, starts, nctx, nblocks, zchunks, s); break;
+        case 2: launch_half<R, SX, SZ, ST, 2>(a, pa, starts, nctx, nblocks, zchunks, s); break;
+        default: launch_half<R, SX, SZ, ST, 3>(a, pa, starts, nctx, nblocks, zchunks, s); break;
         }
     } else if (variant == 2) {
         const int ntx = (a.g.ni + 63) / 64, nty = (a.g.nj + SPLIT_TY - 1) / SPLIT_TY;
@@ -1793,7 +2101,7 @@ static void launch_stage_one(int variant, const StageArgs<R> &a, const StageArgs
 }
 
 template <typename R, int SX, int SZ>
-static void launch_stage_sxz(int variant, int st, const StageArgs<R> &a, const StageArgs<R> *pa, const int *starts,
+void launch_stage_sxz(int variant, int st, const StageArgs<R> &a, const StageArgs<R> *pa, const int *starts,
                              int nctx, int nblocks, int tinc, int rows, int zchunks, hipStream_t s)
 {
     switch (st) {
@@ -1803,6 +2111,38 @@ static void launch_stage_sxz(int variant, int st, const StageArgs<R> &a, const S
     default: launch_stage_one<R, SX, SZ, 3>(variant, a, pa, starts, nctx, nblocks, tinc, rows, zchunks, s); break;
     }
 }
+
+// The stage kernels take most of the compile time: this file is compiled once
+// for every (R, SX, SZ), with CGFD_STAGE_TU naming the one to instantiate
+// (1-8), and once for everything else (0), so that the parts build side by
+// side.
+#define CGFD_STAGE_SXZ(R, SX, SZ)                                                                              \
+    template void launch_stage_sxz<R, SX, SZ>(int, int, const StageArgs<R> &, const StageArgs<R> *, const int *, int, \
+                                              int, int, int, int, hipStream_t);
+#if CGFD_STAGE_TU == 0
+extern CGFD_STAGE_SXZ(float, 1, 1) extern CGFD_STAGE_SXZ(float, 1, -1)
+extern CGFD_STAGE_SXZ(float, -1, 1) extern CGFD_STAGE_SXZ(float, -1, -1)
+extern CGFD_STAGE_SXZ(double, 1, 1) extern CGFD_STAGE_SXZ(double, 1, -1)
+extern CGFD_STAGE_SXZ(double, -1, 1) extern CGFD_STAGE_SXZ(double, -1, -1)
+#elif CGFD_STAGE_TU == 1
+CGFD_STAGE_SXZ(float, 1, 1)
+#elif CGFD_STAGE_TU == 2
+CGFD_STAGE_SXZ(float, 1, -1)
+#elif CGFD_STAGE_TU == 3
+CGFD_STAGE_SXZ(float, -1, 1)
+#elif CGFD_STAGE_TU == 4
+CGFD_STAGE_SXZ(float, -1, -1)
+#elif CGFD_STAGE_TU == 5
+CGFD_STAGE_SXZ(double, 1, 1)
+#elif CGFD_STAGE_TU == 6
+CGFD_STAGE_SXZ(double, 1, -1)
+#elif CGFD_STAGE_TU == 7
+CGFD_STAGE_SXZ(double, -1, 1)
+#elif CGFD_STAGE_TU == 8
+CGFD_STAGE_SXZ(double, -1, -1)
+#endif
+
+#if CGFD_STAGE_TU == 0
 
 template <typename R>
 void launch_stage(int variant, int sx, int sz, int st, const StageArgs<R> &a, const StageArgs<R> *pa, int tinc,
@@ -1923,7 +2263,7 @@ __global__ void step_advance_kernel(int *step)
 
 void launch_step_advance(int *step, hipStream_t s) { step_advance_kernel<<<1, 64, 0, s>>>(step); }
 
-int stage_tile_rows(bool fp64, int tw) { return fp64 ? lds_ty<double>() : lds_ty<float>() * (tw == 32 ? 2 : 1); }
+int stage_tile_rows(bool fp64, int tw) { return HALF_TY * (!fp64 && tw == 32 ? 2 : 1); }
 
 // batched trace gathers: blockIdx.y = grid, whose RecArgs block is
 // kCtxArgBytes from the previous grid's
@@ -1982,5 +2322,7 @@ void launch_step_advance_batch(const char *pa, int nctx, hipStream_t s)
 
 CGFD_INSTANTIATE(float)
 CGFD_INSTANTIATE(double)
+
+#endif // CGFD_STAGE_TU == 0
 
 } // namespace cgfd
