@@ -1681,7 +1681,9 @@ long cgfd_aux_size(const cgfd_ctx *c, int axis)
 static long aux_engine_index(const cgfd_ctx *c, int axis, int pidx, int a, int b)
 {
     // axis 0: (px, y, z); axis 1: (py, x, z); axis 2: (pz, x, y), all 0-based valid
-    if (axis == 0) return ((long)b * c->g.nj + a) * c->npml[0] + pidx;
+    if (axis == 0) // the reference's packed index counts the low side's layers, then the high side's
+        return aux_x_index(c->nabs[0], c->nabs[1], c->g.ni, c->g.nj, c->g.nk,
+                           pidx < c->nabs[0] ? pidx : c->g.ni - c->npml[0] + pidx, a, b);
     if (axis == 1) return ((long)b * c->npml[1] + pidx) * c->g.nxp + a;
     return ((long)pidx * c->g.nj + b) * c->g.nxp + a;
 }

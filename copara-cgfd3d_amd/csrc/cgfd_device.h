@@ -47,6 +47,19 @@ __device__ __forceinline__ long gidx(const Geom &g, int x, int y, int z)
     return g.base + ((long)z * g.nyp + y) * g.nxp + x;
 }
 
+// Element of cell (x, y, z) in an x-axis auxiliary field: the n0 layers of the
+// low side as [z][y][n0], then the n1 of the high side as [z][y][n1].  A tile
+// touches one side only; with both sides in one row its few cells per row
+// would lie n0 + n1 apart, and every row would fetch cache lines that belong
+// mostly to the other side (80-cell rows with 10 + 10 layers: four times the
+// bytes used).
+// A padded field is below 4 GiB, so 32 bits hold the element.
+__host__ __device__ inline unsigned aux_x_index(int n0, int n1, int ni, int nj, int nk, int x, int y, int z)
+{
+    const unsigned row = (unsigned)z * nj + y;
+    return x < n0 ? row * n0 + x : (unsigned)nk * nj * n0 + row * n1 + (x - (ni - n1));
+}
+
 // Correctly rounded s/h for a fixed divisor h, given rh = RN(1/h): one
 // product and a fused remainder correction (Markstein's theorem: with rh the
 // correctly rounded reciprocal and q within one ulp of s/h, q + (s - h q) rh

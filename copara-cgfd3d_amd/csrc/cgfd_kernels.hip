@@ -122,7 +122,7 @@ template <typename AP> __device__ __forceinline__ Geom geom_of(AP a)
 template <typename R> struct Column {
     R APDx, Bx, DBx, APDy, By, DBy;
     bool inx, iny;
-    int ix, iy;
+    int iy;
     unsigned cxy; // element offset of (x,y) inside one [nj][nxp] map
     int col;      // y*ni + x, the source-table column id
 };
@@ -140,7 +140,6 @@ template <typename R, typename AP> __device__ __forceinline__ Column<R> column_o
     k.By = pmy[g.nj + y];
     k.DBy = pmy[2 * g.nj + y];
     k.inx = x < a->nabs[0] || x >= g.ni - a->nabs[1];
-    k.ix = x < a->nabs[0] ? x : x - (g.ni - a->nabs[1]) + a->nabs[0];
     k.iny = y < a->nabs[2] || y >= g.nj - a->nabs[3];
     k.iy = y < a->nabs[2] ? y : y - (g.nj - a->nabs[3]) + a->nabs[2];
     k.cxy = (unsigned)(y * g.nxp + x);
@@ -407,7 +406,7 @@ __device__ __forceinline__ void cell_rates(AP a, const Column<R> &k, const CellI
     }
     if (k.inx) {
         const R APDx = k.APDx, DBx = k.DBx;
-        const long aidx = ((long)z * g.nj + y) * a->npml[0] + k.ix;
+        const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
         AuxIn<R> v;
         load_aux<R, ST>(a, 0, aidx, v);
         R ha[NF];
@@ -949,8 +948,7 @@ __device__ __forceinline__ void half_rates(AP a, const HalfCol<R> &k, const Half
     const unsigned tcell = (unsigned)(top > 0 ? top : 0) * (unsigned)(g.nj * g.nxp) + cxy;
     if (k.inx) {
         const R APDx = k.APDx, DBx = k.DBx;
-        const int ix = x < a->nabs[0] ? x : x - (g.ni - a->nabs[1]) + a->nabs[0];
-        const long aidx = ((long)z * g.nj + y) * a->npml[0] + ix;
+        const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
         HalfAux<R, PART> v;
         load_half_aux<R, ST, PART>(a, 0, aidx, v);
         R ha[NO];
@@ -1577,7 +1575,7 @@ stage_split_kernel(const StageArgs<R> *pa, int tinc)
                 }
             };
             if (k.inx) {
-                const long aidx = ((long)z * g.nj + y) * a->npml[0] + k.ix;
+                const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
                 R ai[NO], ha[NO];
 #pragma unroll
                 for (int c = 0; c < NO; ++c) ai[c] = a->ain[0][(C0 + c) * a->astr[0] + aidx];
@@ -1738,7 +1736,6 @@ __global__ void __launch_bounds__(256) timg_kernel(const TimgArgs<R> av, const T
     const R APDx = pmx[x], Bx = pmx[g.ni + x], DBx = pmx[2 * g.ni + x];
     const R APDy = pmy[y], By = pmy[g.nj + y], DBy = pmy[2 * g.nj + y];
     const bool inx = x < a->nabs[0] || x >= g.ni - a->nabs[1];
-    const int ix = x < a->nabs[0] ? x : x - (g.ni - a->nabs[1]) + a->nabs[0];
     const bool iny = y < a->nabs[2] || y >= g.nj - a->nabs[3];
     const int iy = y < a->nabs[2] ? y : y - (g.nj - a->nabs[3]) + a->nabs[2];
     const double hx = SX > 0 ? a->h : -a->h;
@@ -1840,7 +1837,7 @@ __global__ void __launch_bounds__(256) timg_kernel(const TimgArgs<R> av, const T
             const R DzTz = (R)((double)rhojac * (drp_sum_strf<R, SZ>(vz[m]) / hz));
             R hv = (Bx == (R)1 && By == (R)1) ? DxTx + DyTy + DzTz : DxTx / Bx + DyTy / By + DzTz;
             if (inx) {
-                const R av = a->ain[0][m * a->astr[0] + ((long)z * g.nj + y) * a->npml[0] + ix];
+                const R av = a->ain[0][m * a->astr[0] + aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z)];
                 hv -= av / Bx;
                 a->timg[(3 + m) * a->tstr + tcell] = DBx * DxTx - APDx * av;
             }
