@@ -1066,7 +1066,10 @@ __device__ __forceinline__ void half_sweep(const AP a0, int L, R *ldsbuf)
     const double h = a0->h, rh = a0->rh;
     const unsigned esz = sizeof(R);
     const unsigned plb = (unsigned)(g.plane * esz);
-    const int yc = min(y, g.nyp - 1);
+    // Lanes outside the grid address the guard column ni or the guard row nj,
+    // which are zero like the padding under them, so no line of padding is
+    // fetched.
+    const int xc = min(x, g.ni), yc = min(y, g.nj);
     // Halo slots of this lane.  Rows: wavefront hk stages halo row hk; with two
     // tile rows per wavefront each part of it takes half the components.
     // Columns: the 4*TR slots of a component go to one part of a wavefront;
@@ -1074,8 +1077,8 @@ __device__ __forceinline__ void half_sweep(const AP a0, int L, R *ldsbuf)
     // lane issues the same loads.
     const int hk = wv;
     const int hrow = SX > 0 ? (hk == 0 ? 0 : TR + hk) : (hk < 3 ? hk : TR + 3);
-    const int hy = y0 - O + hrow, hxx = x0 + tx;
-    const bool hv1 = hy >= -3 && hy < g.nyp;
+    const int hy = y0 - O + hrow;
+    const bool hv1 = hy >= 0 && hy < g.nj;
     constexpr int NR = (NIN + HALVES - 1) / HALVES;
 #define CGFD_HALF_FIELD(j) (TW == 64 ? (j) : min(part * NR + (j), NIN - 1))
     constexpr int NH = (NIN + TY * HALVES - 1) / (TY * HALVES);
@@ -1083,15 +1086,15 @@ __device__ __forceinline__ void half_sweep(const AP a0, int L, R *ldsbuf)
     const int hc2k = tx / TR, hr2 = tx % TR;
     const int hcol = SX > 0 ? (hc2k == 0 ? 0 : TW + hc2k) : (hc2k < 3 ? hc2k : TW + 3);
     const int hx2 = x0 - O + hcol, hy2 = y0 + hr2;
-    const bool hv2 = xlane && hx2 >= -3 && hx2 < g.nxp && hy2 < g.nyp;
+    const bool hv2 = xlane && hx2 >= 0 && hx2 < g.ni && hy2 < g.nj;
     auto hfield = [&](int j) { return min(hk + TY * (HALVES * j + part), NIN - 1); };
     auto hkeep = [&](int j) { return xlane && hk + TY * (HALVES * j + part) < NIN; };
-    const int rel_c = (yc * g.nxp + x) * (int)esz;
+    const int rel_c = (yc * g.nxp + xc) * (int)esz;
     const unsigned base0 = (unsigned)(g.base * esz);
     auto pbase = [&](int zz) { return base0 + (unsigned)zz * plb; };
-    // halo slots outside the padded field read offset 0, a guard cell that is
-    // always zero
-    unsigned off1 = hv1 ? pbase(z0) + (hy * g.nxp + hxx) * (int)esz : 0, inc1 = hv1 ? plb : 0;
+    // halo slots outside the grid read offset 0, a guard cell that is always
+    // zero
+    unsigned off1 = hv1 ? pbase(z0) + (hy * g.nxp + xc) * (int)esz : 0, inc1 = hv1 ? plb : 0;
     unsigned off2 = hv2 ? pbase(z0) + (hy2 * g.nxp + hx2) * (int)esz : 0, inc2 = hv2 ? plb : 0;
 
     HalfCol<R> k;
