@@ -213,14 +213,6 @@ static void fb_signs(int t, int k, int *sx, int *sz)
     *sz = (((p == 1 || p == 2) ? 1 : 0) ^ (k & 1)) ? -1 : 1;
 }
 
-// z chunks per column sweep: enough workgroups to fill the chip (~2048
-// 256-cell tiles) and at most ~15 planes per chunk, but at least 2 planes per
-// chunk.  Small grids want many short chunks (64^3: 2.88 -> 4.73
-// Gcell-RKstages/s going from 8 to 2 planes); short chunks also keep the
-// launch's tail short (600x600x300: 6.07 ms per stage with 2 chunks of 150
-// planes, 5.59 ms with 10 of 30; with later kernels 5.338 ms at 10 chunks,
-// 5.328 at 12, 5.305 at 15, 5.300 at 20 and 5.313 at 25; 200x200x150 is
-// fastest at 12 chunks of 13 planes).
 // Tile width of the default stage kernel: the one set or tuned, else 32 when a
 // row of ni cells takes over 8 % more lanes in 64-column tiles than in
 // 32-column ones.  Measured per stage: 80 cells (128 vs 96 lanes) 13 % and
@@ -243,12 +235,23 @@ static long plane_tiles(const cgfd_ctx *c, int tw)
     return (long)((c->g.ni + tw - 1) / tw) * ((c->g.nj + tr - 1) / tr);
 }
 
+// z chunks per column sweep: about 2048 tiles in the launch (4096 workgroups,
+// four rounds of what the chip holds) and at most ~9 planes per chunk.  Short
+// chunks keep the launch's tail short and neighbouring tiles, which share halo
+// lines, close in time; each costs its first window again (4 planes).
+// Measured at 9 / 15 / 30 planes: 200x200x150 357 / 382 / 423 us, 600x600x300
+// 4.78 / 4.81 / 4.87 ms, 32 grids of 80x80x48 per step 4.92 / 4.92 / 5.03 ms.
+// A grid that has at most 2 workgroups per CU with 1 plane each takes 1
+// (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
+// 31.2 us at 1 plane, 29.3 at 2).
+constexpr int kChunkPlanes = 9, kFewBlocks = 512;
 static void default_tuning(cgfd_ctx *c)
 {
     c->rows = 4;
     const long tiles = plane_tiles(c, tile_width(c));
-    long zc = std::max((2048 + tiles - 1) / tiles, (long)(c->g.nk + 14) / 15);
-    zc = std::max(1L, std::min(zc, (long)std::max(1, c->g.nk / 2)));
+    long zc = std::max((2048 + tiles - 1) / tiles, (long)(c->g.nk + kChunkPlanes - 1) / kChunkPlanes);
+    const int least = 2 * tiles * c->g.nk <= kFewBlocks ? 1 : 2; // planes of the shortest chunk
+    zc = std::max(1L, std::min(zc, (long)std::max(1, c->g.nk / least)));
     c->zchunks = (int)zc;
     c->zc_tuned = false;
     c->tile_pref = 0;
@@ -1257,14 +1260,11 @@ static bool batch_fusable(cgfd_ctx *const *ctxs, int n)
 // Workgroups of a batched stage launch (the grids of one tile width tw):
 // every grid sweeps its columns in about the same number of z chunks, chosen
 // for about CGFD_BATCH_WORKGROUPS workgroups over the launch, with at most
-// ~25 and at least 2 planes per chunk per grid; a grid whose z-chunk count
+// ~9 (kChunkPlanes) and at least 2 planes per chunk per grid; a grid whose z-chunk count
 // was tuned (cgfd_autotune, cgfd_set_tuning) keeps its own.  zlen[c] is grid
 // c's chunk length, starts[c] its first workgroup.
 #ifndef CGFD_BATCH_WORKGROUPS
 #define CGFD_BATCH_WORKGROUPS 2048
-#endif
-#ifndef CGFD_BATCH_PLANES
-#define CGFD_BATCH_PLANES 25 // at most about this many planes per chunk
 #endif
 static void batch_layout(cgfd_ctx *const *ctxs, int n, int tw, int *zlen, int *starts)
 {
@@ -1275,7 +1275,7 @@ static void batch_layout(cgfd_ctx *const *ctxs, int n, int tw, int *zlen, int *s
     for (int i = 0; i < n; i++) {
         const int nk = ctxs[i]->g.nk;
         const int zci = ctxs[i]->zc_tuned ? std::max(1, std::min(ctxs[i]->zchunks, nk))
-                                          : (int)std::min(std::max(zc, (long)(nk + CGFD_BATCH_PLANES - 1) / CGFD_BATCH_PLANES),
+                                          : (int)std::min(std::max(zc, (long)(nk + kChunkPlanes - 1) / kChunkPlanes),
                                                           (long)std::max(1, nk / 2));
         zlen[i] = (nk + zci - 1) / zci;
         starts[i + 1] = starts[i] + (int)(plane_tiles(ctxs[i], tw) * zci);
