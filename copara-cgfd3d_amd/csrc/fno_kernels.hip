@@ -47,6 +47,10 @@ struct GemmArgs {
     int act;           // CGFD_FNO_ACT_*
     unsigned short *Cb; // bf16 copy of the result, (m, n) at Cb + z*sEz + m*sEm + n, or null
     long sEz, sEm;
+    // VEC = 2: the result goes to Cb alone, with each index split in two,
+    // (z/zq)*sEz1 + (z%zq)*sEz + (m/mq)*sEm1 + (m%mq)*sEm + (n/nq)*sEn1 + n%nq
+    int zq, mq, nq;
+    long sEz1, sEm1, sEn1;
 };
 
 // One lane's share of a 64 x 32 operand tile (rows r0.., k0..) whose element
@@ -127,7 +131,8 @@ __device__ __forceinline__ float gelu_grad(float x)
 // VEC = 1 every epilogue stream moves 16 bytes per lane (bf16: 8), and the
 // addend is fetched before the K loop.  That layer: 62 -> 44 us (4.2 TB/s);
 // 262144 rows with residual and GELU 110 -> 56 us.  VEC = 0 takes any
-// alignment, element by element.
+// alignment, element by element.  VEC = 2 stores the product in bf16 only, at
+// an address split by index (the spectral layer's transposes).
 template <int AM, int BMODE, int VEC>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 {
@@ -136,19 +141,19 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
     const int z = blockIdx.z, m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     const unsigned short *A = g.A + z * g.sAz;
     const unsigned short *B = g.B + z * g.sBz;
-    float *C = g.C + z * g.sCz;
+    float *C = VEC == 2 ? nullptr : g.C + z * g.sCz;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     f32x4 acc[2][2];
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float *D = g.D ? g.D + z * g.sDz : nullptr;
-    float *pre = g.pre ? g.pre + z * g.sCz : nullptr;
-    unsigned short *Cb = g.Cb ? g.Cb + z * g.sEz : nullptr;
+    const float *D = VEC != 2 && g.D ? g.D + z * g.sDz : nullptr;
+    float *pre = VEC != 2 && g.pre ? g.pre + z * g.sCz : nullptr;
+    unsigned short *Cb = VEC == 2 ? g.Cb + (z / g.zq) * g.sEz1 + (z % g.zq) * g.sEz : g.Cb ? g.Cb + z * g.sEz : nullptr;
     // lane l holds row l%16 and columns 4*(l/16) .. +3 of each 16x16 block
     const int mr = m0 + wm + (lane & 15), nc = n0 + wn + (lane >> 4) * 4;
     f32x4 dv[2][2];
-    if (VEC) {
+    if (VEC == 1) {
 #pragma unroll
         for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
@@ -192,7 +197,14 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj) {
             const int m = mr + bi * 16, n = nc + bj * 16;
-            if (VEC) {
+            if (VEC == 2) {
+                if (m >= g.M || n >= g.N) continue; // N and nq are multiples of 4
+                u16x4 e;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) e[i] = to_bf16(acc[bi][bj][i]);
+                *reinterpret_cast<u16x4 *>(Cb + (m / g.mq) * g.sEm1 + (m % g.mq) * g.sEm + (n / g.nq) * g.sEn1 +
+                                           n % g.nq) = e;
+            } else if (VEC == 1) {
                 if (m >= g.M || n >= g.N) continue; // N is a multiple of 4
                 f32x4 v = acc[bi][bj];
                 if (g.accumulate) v = *reinterpret_cast<const f32x4 *>(C + m * g.sCm + n) + v;
@@ -231,7 +243,8 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 template <int AM, int BMODE>
 void launch_v(const GemmArgs &g, dim3 grid, hipStream_t s)
 {
-    if (g.vec) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 1>), grid, dim3(256), 0, s, g);
+    if (g.vec == 2) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 2>), grid, dim3(256), 0, s, g);
+    else if (g.vec) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 1>), grid, dim3(256), 0, s, g);
     else hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 0>), grid, dim3(256), 0, s, g);
 }
 
@@ -261,6 +274,237 @@ int stage_mode(const void *p, long sZ, long sR, long sK)
     return STAGE_ANY;
 }
 
+void launch_gemm(const GemmArgs &g, int batch, hipStream_t s)
+{
+    const dim3 grid((unsigned)((g.N + BN - 1) / BN), (unsigned)((g.M + BM - 1) / BM), (unsigned)batch);
+    if (g.amode == STAGE_K) launch_b<STAGE_K>(g, grid, s);
+    else if (g.amode == STAGE_MN) launch_b<STAGE_MN>(g, grid, s);
+    else launch_b<STAGE_ANY>(g, grid, s);
+}
+
+// One operand of a product inside a layer: element (r, k) of batch z at
+// p + z*sz + r*sr + k*sk.
+struct Operand {
+    const void *p;
+    long sz, sr, sk;
+};
+
+// Where a bf16-only product goes: plain rows of n, or an address split by index.
+struct Place {
+    void *p;
+    int zq, mq, nq;
+    long sz1, sz, sm1, sm, sn1;
+};
+
+Place rows(void *p, long sz, long sm) { return {p, 1 << 30, 1 << 30, 1 << 30, 0, sz, 0, sm, 0}; }
+
+// bf16-only product; N and every stride and split of the place are multiples
+// of 4, its base aligned to 8 bytes
+void product_bf16(Operand a, Operand b, Place c, int M, int N, int K, int batch, hipStream_t s)
+{
+    GemmArgs g{};
+    g.A = (const unsigned short *)a.p;
+    g.B = (const unsigned short *)b.p;
+    g.sAz = a.sz;
+    g.sAm = a.sr;
+    g.sAk = a.sk;
+    g.sBz = b.sz;
+    g.sBn = b.sr;
+    g.sBk = b.sk;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.amode = stage_mode(a.p, a.sz, a.sr, a.sk);
+    g.bmode = stage_mode(b.p, b.sz, b.sr, b.sk);
+    g.vec = 2;
+    g.Cb = (unsigned short *)c.p;
+    g.zq = c.zq;
+    g.mq = c.mq;
+    g.nq = c.nq;
+    g.sEz1 = c.sz1;
+    g.sEz = c.sz;
+    g.sEm1 = c.sm1;
+    g.sEm = c.sm;
+    g.sEn1 = c.sn1;
+    launch_gemm(g, batch, s);
+}
+
+// The realified mode-mixing weights [[re, im], [-im, re]] of every mode in bf16
+// (p, 2C x 2C), from fp32 (p, C x C) each; and, from block nspec on, the nw
+// pointwise weights in bf16.  Four elements per lane; C is a multiple of 4.
+__global__ void __launch_bounds__(256) layer_weights_kernel(const float *__restrict__ re, const float *__restrict__ im,
+                                                            unsigned short *__restrict__ wr, long nspec4, int C,
+                                                            const float *__restrict__ w,
+                                                            unsigned short *__restrict__ wb, int nw, int nspec)
+{
+    if ((int)blockIdx.x >= nspec) {
+        const int i = (blockIdx.x - nspec) * 256 + threadIdx.x;
+        if (i < nw) wb[i] = to_bf16(w[i]);
+        return;
+    }
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= nspec4) return;
+    const f32x4 a = reinterpret_cast<const f32x4 *>(re)[q], b = reinterpret_cast<const f32x4 *>(im)[q];
+    const long row = q * 4 / C; // p * C + i
+    const int j = (int)(q * 4 % C);
+    const long p = row / C;
+    const int i = (int)(row % C);
+    u16x4 r, c, n;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        r[k] = to_bf16(a[k]);
+        c[k] = to_bf16(b[k]);
+        n[k] = to_bf16(-b[k]);
+    }
+    unsigned short *o = wr + p * 4 * C * C;
+    *reinterpret_cast<u16x4 *>(o + (long)i * 2 * C + j) = r;
+    *reinterpret_cast<u16x4 *>(o + (long)i * 2 * C + C + j) = c;
+    *reinterpret_cast<u16x4 *>(o + (long)(C + i) * 2 * C + j) = n;
+    *reinterpret_cast<u16x4 *>(o + (long)(C + i) * 2 * C + C + j) = r;
+}
+
+// gradients of the two parts from that of the realified weights
+__global__ void __launch_bounds__(256) layer_weight_grads_kernel(const float *__restrict__ gw, float *__restrict__ gre,
+                                                                 float *__restrict__ gim, long nspec4, int C)
+{
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= nspec4) return;
+    const long row = q * 4 / C, p = row / C;
+    const int j = (int)(q * 4 % C), i = (int)(row % C);
+    const float *o = gw + p * 4 * C * C;
+    const f32x4 rr = *reinterpret_cast<const f32x4 *>(o + (long)i * 2 * C + j);
+    const f32x4 ri = *reinterpret_cast<const f32x4 *>(o + (long)i * 2 * C + C + j);
+    const f32x4 ir = *reinterpret_cast<const f32x4 *>(o + (long)(C + i) * 2 * C + j);
+    const f32x4 ii = *reinterpret_cast<const f32x4 *>(o + (long)(C + i) * 2 * C + C + j);
+    reinterpret_cast<f32x4 *>(gre)[q] = rr + ii;
+    reinterpret_cast<f32x4 *>(gim)[q] = ri - ir;
+}
+
+// Backward of a layer's epilogue over a block of GROUP rows of N columns: gz =
+// gy * GELU'(pre) (pre null: gz = gy), its bf16 copy, gz itself on request, and
+// the block's column sums, which the bias gradient adds up.  Each lane keeps V
+// columns (N a multiple of V, N/V at most 256), so the sums cost no second pass
+// over gz.  Bound by HBM: 204800 x 64 with GELU 25 us (5.2 TB/s) without gz,
+// where the GELU backward (38 us) and the sums (22 us) were two passes.
+constexpr int GROUP = 128;
+template <int V>
+__global__ void __launch_bounds__(256) layer_grad_kernel(const float *__restrict__ gy, const float *__restrict__ pre,
+                                                         float *__restrict__ gz, unsigned short *__restrict__ gzb,
+                                                         float *__restrict__ sums, long R, int N)
+{
+    typedef float fv __attribute__((ext_vector_type(V)));
+    typedef unsigned short uv __attribute__((ext_vector_type(V)));
+    __shared__ fv part[256];
+    const int cols = N / V, per = 256 / cols; // rows in flight
+    const int tid = threadIdx.x, c = tid % cols, r = tid / cols;
+    const long r0 = (long)blockIdx.x * GROUP, r1 = r0 + GROUP < R ? r0 + GROUP : R;
+    fv sum = 0.f;
+    if (r < per)
+        for (long i = r0 + r; i < r1; i += per) {
+            const long o = i * cols + c;
+            fv v = reinterpret_cast<const fv *>(gy)[o];
+            if (pre) {
+                const fv x = reinterpret_cast<const fv *>(pre)[o];
+#pragma unroll
+                for (int j = 0; j < V; ++j) v[j] = v[j] * gelu_grad(x[j]);
+            }
+            uv e;
+#pragma unroll
+            for (int j = 0; j < V; ++j) e[j] = to_bf16(v[j]);
+            reinterpret_cast<uv *>(gzb)[o] = e;
+            if (gz) reinterpret_cast<fv *>(gz)[o] = v;
+            sum = sum + v;
+        }
+    part[tid] = sum;
+    __syncthreads();
+    if (tid < cols) {
+        for (int k = 1; k < per; ++k) sum = sum + part[tid + k * cols];
+        reinterpret_cast<fv *>(sums)[(long)blockIdx.x * cols + tid] = sum;
+    }
+}
+
+// out[i] = sum over n of part[n][i] for the weight gradient (first blocks) and
+// the bias gradient, summed in double.  1024 lanes: 64 columns, 16 slices.
+__global__ void __launch_bounds__(1024) layer_reduce_kernel(const float *__restrict__ wpart, int nw, int W,
+                                                            float *__restrict__ gw, const float *__restrict__ bpart,
+                                                            int nb, int N, float *__restrict__ gb, int wblocks)
+{
+    __shared__ double acc[16][64];
+    const bool isw = (int)blockIdx.x < wblocks;
+    const float *src = isw ? wpart : bpart;
+    const int n = isw ? nw : nb, len = isw ? W : N;
+    const int c = (isw ? blockIdx.x : blockIdx.x - wblocks) * 64 + threadIdx.x % 64, sl = threadIdx.x / 64;
+    double s = 0.0;
+    if (c < len) {
+#pragma unroll 4
+        for (int k = sl; k < n; k += 16) s += (double)src[(long)k * len + c];
+    }
+    acc[sl][threadIdx.x % 64] = s;
+    __syncthreads();
+    if (sl == 0 && c < len) {
+        for (int k = 1; k < 16; ++k) s += acc[k][threadIdx.x];
+        (isw ? gw : gb)[c] = (float)s;
+    }
+}
+
+// rows of x and gz that one partial weight-gradient product covers
+constexpr int WROWS = 256;
+
+// Gradients of y = x w + b after its epilogue: gzb and (optional) gz from gy
+// and pre, gw and gb.  wpart: ceil(R/WROWS) x K x N, bpart: ceil(R/GROUP) x N.
+void linear_grads(const float *gy, const float *pre, const void *xb, float *gz, void *gzb, float *wpart, float *bpart,
+                  float *gw, float *gb, long R, int K, int N, hipStream_t s)
+{
+    const int nb = (int)((R + GROUP - 1) / GROUP), nw = (int)((R + WROWS - 1) / WROWS), full = (int)(R / WROWS);
+    if (N % 4 == 0 && vec4(gy, 0, 0, 4) && vec4(pre, 0, 0, 4) && vec4(gz, 0, 0, 4) && vec4(gzb, 0, 0, 2) &&
+        vec4(bpart, 0, 0, 4))
+        hipLaunchKernelGGL(layer_grad_kernel<4>, dim3(nb), dim3(256), 0, s, gy, pre, gz, (unsigned short *)gzb, bpart,
+                           R, N);
+    else
+        hipLaunchKernelGGL(layer_grad_kernel<1>, dim3(nb), dim3(256), 0, s, gy, pre, gz, (unsigned short *)gzb, bpart,
+                           R, N);
+    auto part = [&](long r0, int rows_, int batch, float *out) {
+        GemmArgs g{};
+        g.A = (const unsigned short *)xb + r0 * K;
+        g.B = (const unsigned short *)gzb + r0 * N;
+        g.C = out;
+        g.sAz = (long)WROWS * K;
+        g.sAm = 1;
+        g.sAk = K;
+        g.sBz = (long)WROWS * N;
+        g.sBk = N;
+        g.sBn = 1;
+        g.sCz = (long)K * N;
+        g.sCm = N;
+        g.M = K;
+        g.N = N;
+        g.K = rows_;
+        g.amode = stage_mode(g.A, g.sAz, g.sAm, g.sAk);
+        g.bmode = stage_mode(g.B, g.sBz, g.sBn, g.sBk);
+        g.vec = vec4(out, g.sCz, g.sCm, 4);
+        for (int z = 0; z < batch; z += 65535) { // grid.z
+            GemmArgs h = g;
+            h.A += z * g.sAz;
+            h.B += z * g.sBz;
+            h.C += z * g.sCz;
+            launch_gemm(h, batch - z < 65535 ? batch - z : 65535, s);
+        }
+    };
+    if (full) part(0, WROWS, full, wpart);
+    if (nw > full) part((long)full * WROWS, (int)(R - (long)full * WROWS), 1, wpart + (long)full * K * N);
+    const int wblocks = (K * N + 63) / 64;
+    hipLaunchKernelGGL(layer_reduce_kernel, dim3(wblocks + (N + 63) / 64), dim3(1024), 0, s, wpart, nw, K * N, gw,
+                       bpart, nb, N, gb, wblocks);
+}
+
+int check_layer(long B, long H, long W, long C, long m)
+{
+    if (B <= 0 || H <= 0 || W <= 0 || C <= 0 || m <= 0 || 2 * m > H || m > W / 2) return CGFD_FNO_EINVAL;
+    // vector stores need the width in multiples of 8; grid.z and grid.y limits
+    if (C % 8 != 0 || C > 256 || B * H > 65535 || 2 * m * m > 65535 || B > 65535 || B * H * W > 0x7fffffffL)
+        return CGFD_FNO_EINVAL;
+    return 0;
+}
 
 // gx may alias gy: each element is read before it is written, by one lane.
 // Bound by HBM (14 bytes per element); VEC = 1 moves 4 elements per lane and
@@ -366,14 +610,11 @@ extern "C" int cgfd_fno_gemm_bf16_ex(const void *A, long sAz, long sAm, long sAk
                M, N, K, accumulate ? 1 : 0, stage_mode(A, sAz, sAm, sAk), stage_mode(B, sBz, sBn, sBk),
                N % 4 == 0 && vec4(C, sCz, sCm, 4) && vec4(pre, sCz, sCm, 4) && vec4(D, sDz, sDm, 4) &&
                    vec4(bias, 0, 0, 4) && vec4(C_bf16, sEz, sEm, 2),
-               bias, D, sDz, sDm, pre, act, (unsigned short *)C_bf16, sEz, sEm};
-    const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)batch);
-    const hipStream_t s = (hipStream_t)stream;
-    if (g.amode == STAGE_K) launch_b<STAGE_K>(g, grid, s);
-    else if (g.amode == STAGE_MN) launch_b<STAGE_MN>(g, grid, s);
-    else launch_b<STAGE_ANY>(g, grid, s);
+               bias, D, sDz, sDm, pre, act, (unsigned short *)C_bf16, sEz, sEm, 1, 1, 1, 0, 0, 0};
+    launch_gemm(g, batch, (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
 }
+
 
 extern "C" int cgfd_fno_gemm_bf16(const void *A, long sAz, long sAm, long sAk, const void *B, long sBz, long sBk,
                                   long sBn, float *C, long sCz, long sCm, int M, int N, int K, int batch,
@@ -410,5 +651,89 @@ extern "C" int cgfd_fno_adam(const long long *tensors, const long long *chunks, 
     hipLaunchKernelGGL(adam_kernel, dim3((unsigned)nchunks), dim3(256), 0, (hipStream_t)stream, tensors, chunks,
                        (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)(lr / bc1),
                        (float)__builtin_sqrt(bc2), (float)eps, clear_grad ? 1 : 0);
+    return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
+}
+
+// One Fourier layer, y = act(v w + b + K v).  The spectral branch K v is six
+// launches with bf16 operands throughout: the weights, the DFT along w, that
+// along h (stored mode by mode), the mode mixing (stored back to rows), and
+// the two inverse DFTs.  Every intermediate is a product summed in fp32 and
+// rounded to bf16 once, as the operand of the next product.
+extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
+{
+    if (!L) return CGFD_FNO_EINVAL;
+    const int B = L->B, H = L->H, W = L->W, C = L->C, m = L->modes, P = 2 * m * m;
+    int rc = check_layer(B, H, W, C, m);
+    if (rc) return rc;
+    if (!L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wre || !L->wim || !L->w || !L->bias || !L->wr || !L->wb ||
+        !L->t1 || !L->x || !L->t2 || !L->t3 || !L->sp || !L->y || !L->yb)
+        return CGFD_FNO_EINVAL;
+    const hipStream_t s = (hipStream_t)stream;
+    const long mC = (long)m * C, C2 = 2L * C;
+    const long n4 = (long)P * C * C / 4;
+    const int nspec = (int)((n4 + 255) / 256);
+    hipLaunchKernelGGL(layer_weights_kernel, dim3(nspec + (C * C + 255) / 256), dim3(256), 0, s, L->wre, L->wim,
+                       (unsigned short *)L->wr, n4, C, L->w, (unsigned short *)L->wb, C * C, nspec);
+    // t1 [(b,h)][(ri,kw)][c]
+    product_bf16({L->fw, 0, W, 1}, {L->vb, (long)W * C, 1, C}, rows(L->t1, 2 * mC, C), 2 * m, C, W, B * H, s);
+    // x [(kh,kw)][b][(ri,c)] from rows (ri,kh), columns (kw,c)
+    product_bf16({L->gh, 0, 2L * H, 1}, {L->t1, 2 * H * mC, 1, mC},
+                 {L->x, 1 << 30, 2 * m, C, 0, C2, C, m * B * C2, B * C2}, 4 * m, m * C, 2 * H, B, s);
+    // t2 [b][(kh,ri)][(kw,c)] from batch (kh,kw), rows b, columns (ri,c)
+    product_bf16({L->x, B * C2, C2, 1}, {L->wr, C2 * C2, 1, C2},
+                 {L->t2, m, 1 << 30, C, 2 * mC, C, 0, 4 * m * mC, mC}, B, 2 * C, 2 * C, P, s);
+    // t3 [b][(h,ri)][(kw,c)]
+    product_bf16({L->gi, 0, 4L * m, 1}, {L->t2, 4 * m * mC, 1, mC}, rows(L->t3, 2 * H * mC, mC), 2 * H, m * C, 4 * m, B,
+                 s);
+    rc = cgfd_fno_gemm_bf16(L->fi, 0, 2 * m, 1, L->t3, 2 * mC, C, 1, L->sp, (long)W * C, C, W, C, 2 * m, B * H, 0,
+                            stream);
+    if (rc) return rc;
+    return cgfd_fno_gemm_bf16_ex(L->vb, 0, C, 1, L->wb, 0, C, 1, L->y, 0, C, B * H * W, C, C, 1, 0, L->bias, L->sp, 0, C,
+                                 L->pre, L->gelu ? CGFD_FNO_ACT_GELU : CGFD_FNO_ACT_NONE, L->yb, 0, C, stream);
+}
+
+extern "C" int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *L, void *stream)
+{
+    if (!L) return CGFD_FNO_EINVAL;
+    const int B = L->B, H = L->H, W = L->W, C = L->C, m = L->modes, P = 2 * m * m;
+    int rc = check_layer(B, H, W, C, m);
+    if (rc) return rc;
+    if (!L->gy || !L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wr || !L->wb || !L->x || !L->gzb || !L->t1 ||
+        !L->g || !L->t2 || !L->t3 || !L->gwr || !L->wpart || !L->bpart || !L->gv || !L->gwre || !L->gwim || !L->gw ||
+        !L->gb)
+        return CGFD_FNO_EINVAL;
+    const hipStream_t s = (hipStream_t)stream;
+    const long mC = (long)m * C, C2 = 2L * C, R = (long)B * H * W;
+    linear_grads(L->gy, L->pre, L->vb, nullptr, L->gzb, L->wpart, L->bpart, L->gw, L->gb, R, C, C, s);
+    // transposes of the forward products, from the last to the first
+    product_bf16({L->fi, 0, 1, 2L * m}, {L->gzb, (long)W * C, 1, C}, rows(L->t1, 2 * mC, C), 2 * m, C, W, B * H, s);
+    // g [(kh,kw)][b][(ri,c)] from rows (kh,ri), columns (kw,c)
+    product_bf16({L->gi, 0, 1, 4L * m}, {L->t1, 2 * H * mC, 1, mC},
+                 {L->g, 1 << 30, 2, C, 0, C2, m * B * C2, C, B * C2}, 4 * m, m * C, 2 * H, B, s);
+    // t2 [b][(ri,kh)][(kw,c)] from batch (kh,kw), rows b, columns (ri,c)
+    product_bf16({L->g, B * C2, C2, 1}, {L->wr, C2 * C2, C2, 1},
+                 {L->t2, m, 1 << 30, C, mC, C, 0, 4 * m * mC, 2 * m * mC}, B, 2 * C, 2 * C, P, s);
+    rc = cgfd_fno_gemm_bf16(L->x, B * C2, 1, C2, L->g, B * C2, C2, 1, L->gwr, C2 * C2, C2, 2 * C, 2 * C, B, P, 0, stream);
+    if (rc) return rc;
+    const long n4 = (long)P * C * C / 4;
+    hipLaunchKernelGGL(layer_weight_grads_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, L->gwr, L->gwre,
+                       L->gwim, n4, C);
+    product_bf16({L->gh, 0, 1, 2L * H}, {L->t2, 4 * m * mC, 1, mC}, rows(L->t3, 2 * H * mC, mC), 2 * H, m * C, 4 * m, B,
+                 s);
+    rc = cgfd_fno_gemm_bf16(L->fw, 0, 1, W, L->t3, 2 * mC, C, 1, L->gv, (long)W * C, C, W, C, 2 * m, B * H, 0, stream);
+    if (rc) return rc;
+    return cgfd_fno_gemm_bf16(L->gzb, 0, C, 1, L->wb, 0, 1, C, L->gv, 0, C, (int)R, C, C, 1, 1, stream);
+}
+
+extern "C" int cgfd_fno_linear_bwd(const float *gy, const float *pre, const void *xb, const void *wb, float *gz,
+                                   void *gzb, float *wpart, float *bpart, float *gx, float *gw, float *gb, long R,
+                                   int K, int N, void *stream)
+{
+    if (!gy || !xb || !wb || !gzb || !wpart || !bpart || !gw || !gb || R <= 0 || K <= 0 || N <= 0 || N > 256 ||
+        R > 0x7fffffffL || (R + BM - 1) / BM > 65535 || (K + BM - 1) / BM > 65535)
+        return CGFD_FNO_EINVAL;
+    const hipStream_t s = (hipStream_t)stream;
+    linear_grads(gy, pre, xb, gz, gzb, wpart, bpart, gw, gb, R, K, N, s);
+    if (gx) return cgfd_fno_gemm_bf16(gzb, 0, N, 1, wb, 0, 1, N, gx, 0, K, (int)R, K, N, 1, 0, stream);
     return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
 }

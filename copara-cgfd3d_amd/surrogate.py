@@ -64,7 +64,10 @@ def load_library():
                                               P, L, L, P]
         lib.cgfd_fno_gelu_bwd.argtypes = [P, P, P, P, L, P]
         lib.cgfd_fno_adam.argtypes = [P, P, I, D, D, D, D, LL, I, P]
-        for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam"):
+        lib.cgfd_fno_linear_bwd.argtypes = [P] * 11 + [L, I, I, P]
+        lib.cgfd_fno_fourier_fwd.argtypes = lib.cgfd_fno_fourier_bwd.argtypes = [P, P]
+        for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam",
+                   "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd"):
             getattr(lib, fn).restype = I
         _LIB = lib
     return _LIB
@@ -209,14 +212,27 @@ class _Matmul(torch.autograd.Function):
         return gx[:, :ctx.k], _weight_grad(xb, gyb)[:ctx.k]
 
 
+WROWS, GROUP = 256, 128  # rows per partial sum of a layer's weight and bias gradients (cgfd_fno_linear_bwd)
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
 class _Linear(torch.autograd.Function):
     """y = act(x @ w + b (+ d)) with x [R, K], w [K, N], b [N] and an
     optional residual d [R, N]: one product with the bias, the residual and
-    the GELU in its epilogue.  The backward runs the GELU derivative as one
-    kernel that also writes the bf16 operand of the two gradient products."""
+    the GELU in its epilogue.  The backward is one native call: the GELU
+    derivative with the bf16 operand of the two gradient products and the
+    bias gradient's column sums in one pass, then the products.  keep: the
+    value before the GELU is stored for the backward."""
 
     @staticmethod
-    def forward(ctx, x, w, b, d, gelu, xb, want_bf16):
+    def forward(ctx, x, w, b, d, gelu, xb, want_bf16, keep):
         K = x.shape[1]
         pad = -K % 8
         if xb is None or pad:  # a producer's bf16 copy serves as the operand when no padding is needed
@@ -224,7 +240,7 @@ class _Linear(torch.autograd.Function):
         xb = xb.contiguous()
         wb = torch.nn.functional.pad(w.to(torch.bfloat16), (0, 0, 0, pad)).contiguous()
         y = torch.empty(x.shape[0], w.shape[1], device=x.device, dtype=torch.float32)
-        pre = torch.empty_like(y) if gelu else None
+        pre = torch.empty_like(y) if gelu and keep else None
         yb = torch.empty(y.shape, device=x.device, dtype=torch.bfloat16) if want_bf16 else None
         gemm(xb, wb, y, bias=b.contiguous(), addend=None if d is None else d.contiguous(), pre=pre,
              act=ACT_GELU if gelu else ACT_NONE, out_bf16=yb)
@@ -240,13 +256,107 @@ class _Linear(torch.autograd.Function):
     def backward(ctx, gy, *unused):
         xb, wb, pre = ctx.saved_tensors
         gy = gy.contiguous()
+        (R, K), N, dev = xb.shape, wb.shape[1], gy.device
+        if N > 256 or not gy.is_cuda or gy.dtype != torch.float32:
+            return _Linear._backward_parts(ctx, gy, xb, wb, pre)
+        new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+        gz = new(R, N) if ctx.has_d and ctx.gelu else None
+        gzb, gx = new(R, N, dtype=torch.bfloat16), new(R, K) if ctx.needs_input_grad[0] else None
+        gw, gb, wpart, bpart = new(K, N), new(N), new(-(-R // WROWS) * K * N), new(-(-R // GROUP) * N)
+        rc = load_library().cgfd_fno_linear_bwd(_ptr(gy), _ptr(pre), _ptr(xb), _ptr(wb), _ptr(gz), _ptr(gzb),
+                                                _ptr(wpart), _ptr(bpart), _ptr(gx), _ptr(gw), _ptr(gb), R, K, N,
+                                                _stream())
+        if rc != 0:
+            raise SurrogateError(f"cgfd_fno_linear_bwd returned {rc}")
+        gd = (gz if ctx.gelu else gy) if ctx.has_d else None
+        return None if gx is None else gx[:, :ctx.k], gw[:ctx.k], gb, gd, None, None, None, None
+
+    @staticmethod
+    def _backward_parts(ctx, gy, xb, wb, pre):
+        """The same from single products, for more than 256 columns."""
         if ctx.gelu:
             gz, gzb = gelu_backward(gy, pre)
         else:
             gz, gzb = gy, gy.to(torch.bfloat16)
         gx = torch.empty(xb.shape, device=gy.device, dtype=torch.float32)
         gemm(gzb, wb.t(), gx)
-        return gx[:, :ctx.k], _weight_grad(xb, gzb)[:ctx.k], gz.sum(0), (gz if ctx.has_d else None), None, None, None
+        return (gx[:, :ctx.k], _weight_grad(xb, gzb)[:ctx.k], gz.sum(0), (gz if ctx.has_d else None), None, None, None,
+                None)
+
+
+class _Forward(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_int) for n in ("B", "H", "W", "C", "modes", "gelu")] +
+                [(n, ctypes.c_void_p) for n in ("vb", "fw", "gh", "gi", "fi", "wre", "wim", "w", "bias", "wr", "wb", "x",
+                                                "t1", "t2", "t3", "sp", "y", "pre", "yb")])
+
+
+class _Backward(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_int) for n in ("B", "H", "W", "C", "modes", "unused")] +
+                [(n, ctypes.c_void_p) for n in ("gy", "pre", "vb", "fw", "gh", "gi", "fi", "wr", "wb", "x", "gzb", "g",
+                                                "t1", "t2", "t3", "gwr", "wpart", "bpart", "gv", "gwre", "gwim", "gw",
+                                                "gb")])
+
+
+def fused_layer_ok(B, H, W, C, m):
+    """Whether cgfd_fno_fourier_fwd takes a layer of this size (vector stores
+    need the width in multiples of 8; launch limits)."""
+    return (C % 8 == 0 and C <= 256 and B * H <= 65535 and 2 * m * m <= 65535 and 2 * m <= H and m <= W // 2
+            and (B * H * W + 63) // 64 <= 65535)
+
+
+class _FourierLayer(torch.autograd.Function):
+    """y = act(v w + b + K v), one Fourier layer, on the native launches of
+    cgfd_fno_fourier_fwd / _bwd: what _LeftConst, _Bmm and _Linear compute one
+    after another, with the intermediates in bf16 only and no permuted copies.
+    v [R, C] with its bf16 copy vb; returns y and its bf16 copy."""
+
+    @staticmethod
+    def forward(ctx, v, vb, wre, wim, w, b, shape, m, gelu, keep):
+        B, H, W = shape
+        C, dev = v.shape[1], v.device
+        P = 2 * m * m
+        vb = (v.to(torch.bfloat16) if vb is None else vb).contiguous()
+        mats = dft_matrices(H, W, m, dev)
+        wre, wim, w, b = (t.contiguous() for t in (wre, wim, w, b))
+        new = lambda *n, dtype=torch.bfloat16: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+        wr, wb, x = new(P, 2 * C, 2 * C), new(C, C), new(P, B, 2 * C)
+        t1, t2, t3 = new(2 * B * H * m * C), new(4 * B * m * m * C), new(2 * B * H * m * C)
+        sp, y, yb = new(v.shape, dtype=torch.float32), new(v.shape, dtype=torch.float32), new(v.shape)
+        pre = new(v.shape, dtype=torch.float32) if gelu and keep else None
+        arg = _Forward(B, H, W, C, m, int(gelu), _ptr(vb), *(_ptr(t) for t in mats), _ptr(wre), _ptr(wim), _ptr(w),
+                       _ptr(b), _ptr(wr), _ptr(wb), _ptr(x), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(sp), _ptr(y), _ptr(pre),
+                       _ptr(yb))
+        rc = load_library().cgfd_fno_fourier_fwd(ctypes.byref(arg), _stream())
+        if rc != 0:
+            raise SurrogateError(f"cgfd_fno_fourier_fwd returned {rc}")
+        if keep:
+            ctx.save_for_backward(vb, wr, wb, x, pre, *mats)
+        ctx.dims = (B, H, W, C, m)
+        ctx.mark_non_differentiable(yb)
+        ctx.set_materialize_grads(False)
+        return y, yb
+
+    @staticmethod
+    def backward(ctx, gy, *unused):
+        vb, wr, wb, x, pre, *mats = ctx.saved_tensors
+        B, H, W, C, m = ctx.dims
+        R, P, dev = B * H * W, 2 * m * m, gy.device
+        gy = gy.contiguous()
+        if gy.data_ptr() % 16:
+            gy = gy.clone()
+        new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+        bf = torch.bfloat16
+        gzb, g = new(R, C, dtype=bf), new(P, B, 2 * C, dtype=bf)
+        t1, t2, t3 = new(2 * B * H * m * C, dtype=bf), new(4 * B * m * m * C, dtype=bf), new(2 * B * H * m * C, dtype=bf)
+        gwr, wpart, bpart = new(P, 2 * C, 2 * C), new(-(-R // WROWS) * C * C), new(-(-R // GROUP) * C)
+        gv, gwre, gwim, gw, gb = new(R, C), new(P, C, C), new(P, C, C), new(C, C), new(C)
+        arg = _Backward(B, H, W, C, m, 0, _ptr(gy), _ptr(pre), _ptr(vb), *(_ptr(t) for t in mats), _ptr(wr), _ptr(wb),
+                        _ptr(x), _ptr(gzb), _ptr(g), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(gwr), _ptr(wpart), _ptr(bpart),
+                        _ptr(gv), _ptr(gwre), _ptr(gwim), _ptr(gw), _ptr(gb))
+        rc = load_library().cgfd_fno_fourier_bwd(ctypes.byref(arg), _stream())
+        if rc != 0:
+            raise SurrogateError(f"cgfd_fno_fourier_bwd returned {rc}")
+        return gv, None, gwre, gwim, gw, gb, None, None, None, None
 
 
 class _Bmm(torch.autograd.Function):
@@ -414,7 +524,7 @@ def linear(x, w, b, backend, d=None, gelu=False, xb=None, want_bf16=False):
     with want_bf16 the result comes with its own bf16 copy, (y, yb) (yb is
     None on the torch backend)."""
     if backend == "mfma":
-        return _Linear.apply(x, w, b, d, gelu, xb, want_bf16)
+        return _Linear.apply(x, w, b, d, gelu, xb, want_bf16, torch.is_grad_enabled())
     y = x @ w + b
     if d is not None:
         y = y + d
@@ -500,7 +610,12 @@ class FNO2d(torch.nn.Module):
         B, H, W, _ = x.shape
         R = B * H * W
         v, vb = linear(x.reshape(R, -1), self.lift_w, self.lift_b, backend, want_bf16=True)
+        fused = backend == "mfma" and fused_layer_ok(B, H, W, self.width, self.modes)
         for l in range(self.layers):
+            if fused:
+                v, vb = _FourierLayer.apply(v, vb, self.spec_re[l], self.spec_im[l], self.pw_w[l], self.pw_b[l],
+                                            (B, H, W), self.modes, l < self.layers - 1, torch.is_grad_enabled())
+                continue
             sp = self._spectral(v.reshape(B, H, W, self.width), l, backend, vb).reshape(R, self.width)
             v, vb = linear(v, self.pw_w[l], self.pw_b[l], backend, d=sp, gelu=l < self.layers - 1, xb=vb,
                            want_bf16=True)

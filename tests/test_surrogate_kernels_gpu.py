@@ -78,3 +78,70 @@ def test_adam_vector_ends(n):
         assert not p.grad.any()
     # three steps of at most lr each, every operation within an ulp or two
     assert np.abs((p - q).detach().cpu().numpy()).max() <= 3 * (1e-2 * 16 * EPS + 4 * EPS * float(q.detach().abs().max()))
+
+
+# rows below, at and past the partial sums' lengths; 1, 3 and 256 columns, a
+# padded K, no GELU, a residual
+@pytest.mark.parametrize("R,K,N", [(1, 8, 1), (127, 13, 3), (129, 64, 64), (256, 16, 20), (700, 40, 256), (1025, 8, 7)])
+@pytest.mark.parametrize("gelu,residual", [(True, True), (True, False), (False, True)])
+def test_linear_backward_against_single_products(R, K, N, gelu, residual):
+    ins = [_rand((R, K), 1), _rand((K, N), 2), _rand((N,), 3)] + ([_rand((R, N), 4)] if residual else [])
+    gy, got = _rand((R, N), 5).cuda(), []
+    for parts in (False, True):
+        t = [v.cuda().requires_grad_() for v in ins]
+        y = surrogate.linear(*t[:3], "mfma", d=t[3] if residual else None, gelu=gelu)
+        if parts:
+            with pytest.MonkeyPatch.context() as mp:
+                mp.setattr(surrogate._Linear, "backward", staticmethod(_parts_backward))
+                y.backward(gy)
+        else:
+            y.backward(gy)
+        got.append([v.grad for v in t])
+    one, two = got
+    assert torch.equal(one[0], two[0])
+    if residual:
+        assert torch.equal(one[3], two[3])
+    gz = two[3].double().cpu() if residual else None
+    x = ins[0].bfloat16().double()
+    if gz is not None:  # sums of R terms in fp32 against 64 bits
+        b = gz.float().bfloat16().double()
+        assert ((one[1].double().cpu() - x.t() @ b).abs() <= (R + 4) * EPS * (x.abs().t() @ b.abs())).all()
+        assert ((one[2].double().cpu() - gz.sum(0)).abs() <= (R + 4) * EPS * gz.abs().sum(0)).all()
+    else:
+        size = float(x.abs().max()) * float(gy.abs().max()) * 1.2
+        assert (one[1] - two[1]).abs().max() <= 2 * (R + 4) * EPS * R * size
+        assert (one[2] - two[2]).abs().max() <= 2 * (R + 4) * EPS * R * size
+
+
+def _parts_backward(ctx, gy, *unused):
+    return surrogate._Linear._backward_parts(ctx, gy.contiguous(), *ctx.saved_tensors)
+
+
+# rows of the transforms that are no multiple of 8, the smallest width, one
+# mode, a last layer without GELU (layers = 1) and one with it
+@pytest.mark.parametrize("B,H,W,C,m,layers", [(1, 4, 4, 8, 1, 1), (2, 9, 11, 8, 3, 2), (3, 16, 20, 24, 5, 2), (2, 33, 40, 64, 16, 1),
+                                              (5, 12, 26, 40, 6, 3)])
+def test_fourier_layer_against_single_products(B, H, W, C, m, layers, monkeypatch):
+    net = surrogate.FNO2d(surrogate.NCH, 3, C, m, layers, proj=32, seed=3).cuda()
+    assert surrogate.fused_layer_ok(B, H, W, C, m)
+    x, gy = _rand((B, H, W, surrogate.NCH), 1).cuda(), _rand((B, H, W, 3), 2).cuda()
+    got = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(surrogate, "fused_layer_ok", lambda *a: False)
+        net.zero_grad(set_to_none=True)
+        y = net(x)
+        y.backward(gy)
+        with torch.no_grad():
+            assert torch.equal(net(x), y)
+        got.append((y.detach(), {n: p.grad for n, p in net.named_parameters()}))
+    # the same products of the same bf16 operands in the same order; only the
+    # sums over all rows (pointwise weight gradients, and what the unfused
+    # spectral weights share with them) are ordered differently
+    assert torch.equal(got[0][0], got[1][0])
+    for n, g in got[0][1].items():
+        if n.startswith("spec"):
+            assert torch.equal(g, got[1][1][n]), n
+        else:
+            scale = float(g.abs().max()) + 1e-30
+            assert float((g - got[1][1][n]).abs().max()) <= (B * H * W + 4) * EPS * scale, n
