@@ -56,26 +56,32 @@ struct GemmArgs {
 // One lane's share of a 64 x 32 operand tile (rows r0.., k0..) whose element
 // (r, k) sits at P + r*sR + k*sK: eight bf16 values, loaded into registers
 // so that the next tile's loads overlap the current tile's products.
-template <int MODE>
+// EX = 1: no group of eight crosses the operand's edge (K a multiple of 8 in mode
+// K, R in mode MN), so a share is loaded whole or is zero.  The element-wise
+// path for crossing groups takes 30 registers: without it 6-8 instead of 4-5
+// wavefronts fit a SIMD, and a training batch (32 x 80 x 80, width 64) takes 1604
+// instead of 1683 us on the GPU.  Fetching 2 or 3 tiles ahead instead of one
+// gave nothing (1633, 1682 us).
+template <int MODE, int EX>
 __device__ __forceinline__ u16x8 fetch(const unsigned short *P, long sR, long sK, int r0, int k0, int R, int K,
                                        int tid)
 {
-    u16x8 v;
+    u16x8 v = 0;
     if (MODE == STAGE_MN) {
         // 8 consecutive rows at one k
         const int r = r0 + (tid & 7) * 8, k = k0 + (tid >> 3);
-        if (k < K && r + 7 < R) {
+        if (k < K && r + (EX ? 0 : 7) < R) {
             v = *reinterpret_cast<const u16x8 *>(P + r * sR + k * sK);
-        } else {
+        } else if (!EX) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = (k < K && r + i < R) ? P[(r + i) * sR + k * sK] : (unsigned short)0;
         }
     } else {
         // 8 consecutive k of one row
         const int r = r0 + (tid >> 2), k = k0 + (tid & 3) * 8;
-        if (MODE == STAGE_K && r < R && k + 7 < K) {
+        if (MODE == STAGE_K && r < R && k + (EX ? 0 : 7) < K) {
             v = *reinterpret_cast<const u16x8 *>(P + r * sR + k);
-        } else {
+        } else if (MODE == STAGE_ANY || !EX) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = (r < R && k + j < K) ? P[r * sR + (k + j) * sK] : (unsigned short)0;
         }
@@ -133,7 +139,7 @@ __device__ __forceinline__ float gelu_grad(float x)
 // 262144 rows with residual and GELU 110 -> 56 us.  VEC = 0 takes any
 // alignment, element by element.  VEC = 2 stores the product in bf16 only, at
 // an address split by index (the spectral layer's transposes).
-template <int AM, int BMODE, int VEC>
+template <int AM, int BMODE, int VEC, int EX>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 {
     __shared__ __attribute__((aligned(16))) unsigned short As[2][BM][BK + PAD];
@@ -152,6 +158,9 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
     unsigned short *Cb = VEC == 2 ? g.Cb + (z / g.zq) * g.sEz1 + (z % g.zq) * g.sEz : g.Cb ? g.Cb + z * g.sEz : nullptr;
     // lane l holds row l%16 and columns 4*(l/16) .. +3 of each 16x16 block
     const int mr = m0 + wm + (lane & 15), nc = n0 + wn + (lane >> 4) * 4;
+    // A rows are m (stride sAm), B "rows" are n (stride sBn)
+    u16x8 na = fetch<AM, EX>(A, g.sAm, g.sAk, m0, 0, g.M, g.K, tid);
+    u16x8 nb = fetch<BMODE, EX>(B, g.sBn, g.sBk, n0, 0, g.N, g.K, tid);
     f32x4 dv[2][2];
     if (VEC == 1) {
 #pragma unroll
@@ -163,17 +172,15 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
             }
     }
 
-    // A rows are m (stride sAm), B "rows" are n (stride sBn)
-    park<AM>(As[0], fetch<AM>(A, g.sAm, g.sAk, m0, 0, g.M, g.K, tid), tid);
-    park<BMODE>(Bs[0], fetch<BMODE>(B, g.sBn, g.sBk, n0, 0, g.N, g.K, tid), tid);
+    park<AM>(As[0], na, tid);
+    park<BMODE>(Bs[0], nb, tid);
     __syncthreads();
     int cur = 0;
     for (int k0 = 0; k0 < g.K; k0 += BK) {
         const bool more = k0 + BK < g.K;
-        u16x8 na, nb;
         if (more) {
-            na = fetch<AM>(A, g.sAm, g.sAk, m0, k0 + BK, g.M, g.K, tid);
-            nb = fetch<BMODE>(B, g.sBn, g.sBk, n0, k0 + BK, g.N, g.K, tid);
+            na = fetch<AM, EX>(A, g.sAm, g.sAk, m0, k0 + BK, g.M, g.K, tid);
+            nb = fetch<BMODE, EX>(B, g.sBn, g.sBk, n0, k0 + BK, g.N, g.K, tid);
         }
         const int kq = (lane >> 4) * 8;
 #pragma unroll
@@ -243,9 +250,14 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 template <int AM, int BMODE>
 void launch_v(const GemmArgs &g, dim3 grid, hipStream_t s)
 {
-    if (g.vec == 2) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 2>), grid, dim3(256), 0, s, g);
-    else if (g.vec) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 1>), grid, dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 0>), grid, dim3(256), 0, s, g);
+    // whole groups of eight along the staged index of both operands
+    const bool ex = (AM != STAGE_K || g.K % 8 == 0) && (AM != STAGE_MN || g.M % 8 == 0) &&
+                    (BMODE != STAGE_K || g.K % 8 == 0) && (BMODE != STAGE_MN || g.N % 8 == 0);
+    if (g.vec == 2 && ex) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 2, 1>), grid, dim3(256), 0, s, g);
+    else if (g.vec == 2) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 2, 0>), grid, dim3(256), 0, s, g);
+    else if (g.vec && ex) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 1, 1>), grid, dim3(256), 0, s, g);
+    else if (g.vec) hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 1, 0>), grid, dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((gemm_bf16_kernel<AM, BMODE, 0, 0>), grid, dim3(256), 0, s, g);
 }
 
 template <int AM>

@@ -145,3 +145,19 @@ def test_fourier_layer_against_single_products(B, H, W, C, m, layers, monkeypatc
         else:
             scale = float(g.abs().max()) + 1e-30
             assert float((g - got[1][1][n]).abs().max()) <= (B * H * W + 4) * EPS * scale, n
+
+
+# operands staged whole (extents in multiples of 8), groups of eight that cross
+# the edge (60 of 64 columns of a wider buffer), and every pair of layouts
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (72, 136, 40), (60, 60, 60), (8, 8, 8), (100, 20, 76)])
+@pytest.mark.parametrize("at,bt", [(False, False), (True, False), (False, True), (True, True)])
+def test_gemm_staging_at_group_edges(M, N, K, at, bt):
+    def wide(r, c, t, seed):  # r x c inside rows of a multiple of 8
+        full = _rand((c, -(-r // 8) * 8) if t else (r, -(-c // 8) * 8), seed).bfloat16().cuda()
+        return full[:, :r].t() if t else full[:, :c]
+
+    a, b = wide(M, K, at, 1), wide(K, N, bt, 2)
+    out = torch.full((M, N), 7.0, device="cuda")
+    surrogate.gemm(a, b, out)
+    x, y = a.double().cpu(), b.double().cpu()
+    assert ((out.cpu().double() - x @ y).abs() <= (K + 4) * EPS * (x.abs() @ y.abs())).all()
