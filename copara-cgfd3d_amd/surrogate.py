@@ -66,7 +66,8 @@ def load_library():
         lib.cgfd_fno_adam.argtypes = [P, P, I, D, D, D, D, LL, I, P]
         lib.cgfd_fno_linear_bwd.argtypes = [P] * 11 + [L, I, I, P]
         lib.cgfd_fno_fourier_fwd.argtypes = lib.cgfd_fno_fourier_bwd.argtypes = [P, P]
-        for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam",
+        lib.cgfd_fno_encode.argtypes = [P, P, I, I, I, I, I, D, D, P]
+        for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam", "cgfd_fno_encode",
                    "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd"):
             getattr(lib, fn).restype = I
         _LIB = lib
@@ -81,6 +82,16 @@ def _span_ok(t, offsets):
 
 
 ACT_NONE, ACT_GELU = 0, 1
+
+
+def _pad_cols(t, n):
+    """n zero columns on the right (none: t itself, without the copy that
+    torch's pad would make)."""
+    return torch.nn.functional.pad(t, (0, n)) if n else t
+
+
+def _pad_rows(t, n):
+    return torch.nn.functional.pad(t, (0, 0, 0, n)) if n else t
 
 
 def _as3(t):
@@ -195,8 +206,8 @@ class _Matmul(torch.autograd.Function):
     def forward(ctx, x, w):
         K = x.shape[1]
         pad = -K % 8
-        xb = torch.nn.functional.pad(x.to(torch.bfloat16), (0, pad)).contiguous()
-        wb = torch.nn.functional.pad(w.to(torch.bfloat16), (0, 0, 0, pad)).contiguous()
+        xb = _pad_cols(x.to(torch.bfloat16), pad).contiguous()
+        wb = _pad_rows(w.to(torch.bfloat16), pad).contiguous()
         y = torch.empty(x.shape[0], w.shape[1], device=x.device, dtype=torch.float32)
         gemm(xb, wb, y)
         ctx.save_for_backward(xb, wb)
@@ -236,9 +247,9 @@ class _Linear(torch.autograd.Function):
         K = x.shape[1]
         pad = -K % 8
         if xb is None or pad:  # a producer's bf16 copy serves as the operand when no padding is needed
-            xb = torch.nn.functional.pad(x.to(torch.bfloat16), (0, pad))
+            xb = _pad_cols(x.to(torch.bfloat16), pad)
         xb = xb.contiguous()
-        wb = torch.nn.functional.pad(w.to(torch.bfloat16), (0, 0, 0, pad)).contiguous()
+        wb = _pad_rows(w.to(torch.bfloat16), pad).contiguous()
         y = torch.empty(x.shape[0], w.shape[1], device=x.device, dtype=torch.float32)
         pre = torch.empty_like(y) if gelu and keep else None
         yb = torch.empty(y.shape, device=x.device, dtype=torch.bfloat16) if want_bf16 else None
@@ -903,6 +914,24 @@ def encode(base, src):
     return out
 
 
+def encode_device(base, src, device):
+    """encode's fields as a tensor on `device`, computed there when it is a GPU
+    (the same operations in double, rounded once to fp32)."""
+    if torch.device(device).type != "cuda" or not 0 < len(src) <= 65535:
+        return torch.from_numpy(encode(base, src)).to(device)
+    i0, j0, wi, wj = _window(base)
+    rows = torch.from_numpy(np.ascontiguousarray(src, dtype=np.float64)).to(device)
+    if rows.shape[1] != 10:
+        raise SurrogateError("source rows have 10 columns (see source_rows)")
+    out = torch.empty(len(src), wi, wj, NCH, device=device, dtype=torch.float32)
+    with torch.cuda.device(out.device):
+        rc = load_library().cgfd_fno_encode(_ptr(rows), _ptr(out), len(src), i0, j0, wi, wj, float(base["dh"]),
+                                            max(base["ni"], base["nj"]) * base["dh"], _stream())
+    if rc != 0:
+        raise SurrogateError(f"cgfd_fno_encode returned {rc}")
+    return out
+
+
 def target(pgv, src):
     """log10(PGV / M0) [n, ni, nj, 3] of source rows (a floor keeps silent
     points finite)."""
@@ -998,7 +1027,7 @@ class Surrogate:
                 traces = np.concatenate([transform_traces(self.base, traces, g) for g in SYM])
             src = np.concatenate([p[0] for p in pairs])
             pgv = np.concatenate([p[1] for p in pairs])
-        x = torch.from_numpy(encode(self.base, src)).to(self.device)
+        x = encode_device(self.base, src, self.device)
         y = target(pgv, src)
         self.mu, self.sd = float(y.mean()), float(y.std())
         y = torch.from_numpy((y - self.mu) / self.sd).to(self.device)
@@ -1045,7 +1074,7 @@ class Surrogate:
         touts = [0.0 for _ in self.nets]
         for g in images:
             sg, _ = transform(self.base, src, None, g)
-            x = torch.from_numpy(encode(self.base, sg)).to(self.device)
+            x = encode_device(self.base, sg, self.device)
             for k in range(len(self.nets)):
                 parts = [self._outputs(k, x[b:b + batch]) for b in range(0, len(x), batch)]
                 o = torch.cat([p[0] for p in parts])

@@ -98,6 +98,13 @@ int cgfd_fno_linear_bwd(const float *gy, const float *pre, const void *xb, const
  * (the operand of the next backward products).  gx may alias gy. */
 int cgfd_fno_gelu_bwd(const float *gy, const float *pre, float *gx, void *gx_bf16, long n, void *stream);
 
+/* The network's 13 input fields [n, wi, wj, 13] of n sources at the surface
+ * points (i0 + i, j0 + j)*dh: src is n rows of 10 doubles on the device (x, y,
+ * depth, mxx, myy, mzz, mxy, mxz, myz, log10 M0), L the length the coordinates
+ * are scaled by.  n is at most 65535. */
+int cgfd_fno_encode(const double *src, float *out, int n, int i0, int j0, int wi, int wj, double dh, double L,
+                    void *stream);
+
 /* One Adam step (torch.optim.Adam without weight decay or amsgrad) over many
  * fp32 tensors in one launch.  tensors: device array of 5 int64 per tensor
  * (parameter, gradient, first moment, second moment addresses, element

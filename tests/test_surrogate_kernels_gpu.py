@@ -161,3 +161,21 @@ def test_gemm_staging_at_group_edges(M, N, K, at, bt):
     surrogate.gemm(a, b, out)
     x, y = a.double().cpu(), b.double().cpu()
     assert ((out.cpu().double() - x @ y).abs() <= (K + 4) * EPS * (x.abs() @ y.abs())).all()
+
+
+@pytest.mark.parametrize("n,window", [(1, None), (3, 14), (5, 20)])
+def test_encode_on_the_device(n, window):
+    """The same operations in double: equal but for the last bit, where exp
+    and log10 round differently."""
+    base = dict(ni=20, nj=20, dh=100.0)
+    if window:
+        base["window"] = ((20 - window) // 2, (20 - window) // 2, window)
+    rng = np.random.default_rng(n)
+    src = np.concatenate([rng.uniform(0, 2000, (n, 2)), rng.uniform(500, 3000, (n, 1)), rng.uniform(-1, 1, (n, 6)),
+                          rng.uniform(14, 17, (n, 1))], 1)
+    want = surrogate.encode(base, src)
+    got = surrogate.encode_device(base, src, "cuda").cpu().numpy()
+    assert got.shape == want.shape
+    exact = [c for c in range(13) if c not in (4, 7)]
+    assert np.array_equal(got[..., exact], want[..., exact])
+    assert (np.abs(got - want) <= EPS * np.abs(want)).all()
