@@ -489,6 +489,148 @@ __global__ void __launch_bounds__(256) encode_kernel(const double *__restrict__ 
     o[12] = (float)p[8];
 }
 
+// The last step of a Fourier layer in one launch: for every grid row z = (b,h),
+//   forward:  y = act(V W + bias + F T),  pre and the bf16 copy as on request
+//   backward: y = V W + F T
+// with V [W, C] and T [2m, C] of that row and the constant W [C, C], F [W, 2m]
+// (each operand by strides).  Two launches wrote the inverse transform F T in
+// fp32 and read it back.  The two products accumulate apart and are added in the
+// order of those launches, so the results are theirs bit for bit.  A block of
+// 2*WR wavefronts owns 32*WR points of a row by 64 channels, so that 80 or 96
+// points are one block (WR = 3) and 128 are one (WR = 4).  Bound by HBM: 2560 rows
+// of 80 points, 64 channels and 16 modes with every output take 38 us (183 MB
+// moved, 4.8 TB/s) where the two launches took 19 + 39, the backward 28 us for
+// 18 + 24.
+struct PairArgs {
+    const unsigned short *F, *T, *V, *Wt;
+    long sFr, sFk, sTz, sTk, sVz, sVr, sWn, sWk;
+    int M, N, K1, K2, act;
+    const float *bias;
+    float *y, *pre;
+    unsigned short *yb;
+};
+
+template <int WR, int MODE>
+__device__ __forceinline__ u16x8 pair_fetch_a(const unsigned short *P, long sR, long sK, int r0, int k0, int R, int K)
+{
+    const int tid = threadIdx.x;
+    u16x8 v = 0;
+    const int r = r0 + (MODE == STAGE_MN ? tid % (4 * WR) * 8 : tid >> 2);
+    const int k = k0 + (MODE == STAGE_MN ? tid / (4 * WR) : (tid & 3) * 8);
+    if (r < R && k < K) v = *reinterpret_cast<const u16x8 *>(P + r * sR + k * sK);
+    return v;
+}
+
+template <int WR, int MODE>
+__device__ __forceinline__ void pair_park_a(unsigned short (*T)[BK + PAD], u16x8 v)
+{
+    const int tid = threadIdx.x;
+    if (MODE == STAGE_MN) {
+        const int r = tid % (4 * WR) * 8, k = tid / (4 * WR);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) T[r + i][k] = v[i];
+    } else {
+        *reinterpret_cast<u16x8 *>(&T[tid >> 2][(tid & 3) * 8]) = v;
+    }
+}
+
+template <int WR, int BWD>
+__global__ void __launch_bounds__(128 * WR) layer_pair_kernel(PairArgs g)
+{
+    // staging: F rows by k (forward) or by point (its transpose), T by channel,
+    // V by k, W by channel (forward) or by k (its transpose)
+    constexpr int FM = BWD ? STAGE_MN : STAGE_K, WM = BWD ? STAGE_K : STAGE_MN;
+    __shared__ __attribute__((aligned(16))) unsigned short As[2][32 * WR][BK + PAD];
+    __shared__ __attribute__((aligned(16))) unsigned short Bs[2][BN][BK + PAD];
+    const int z = blockIdx.z, m0 = blockIdx.y * 32 * WR, n0 = blockIdx.x * BN;
+    const unsigned short *T = g.T + z * g.sTz, *V = g.V + z * g.sVz;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    f32x4 accF[2][2], accV[2][2];
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) accF[i][j] = accV[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int t1 = (g.K1 + BK - 1) / BK, tiles = t1 + (g.K2 + BK - 1) / BK;
+    const bool loadb = tid < 256;
+    u16x8 na = 0, nb = 0;
+    auto get = [&](int t) {
+        if (t < t1) {
+            na = pair_fetch_a<WR, FM>(g.F, g.sFr, g.sFk, m0, t * BK, g.M, g.K1);
+            if (loadb) nb = fetch<STAGE_MN, 1>(T, 1, g.sTk, n0, t * BK, g.N, g.K1, tid);
+        } else {
+            na = pair_fetch_a<WR, STAGE_K>(V, g.sVr, 1, m0, (t - t1) * BK, g.M, g.K2);
+            if (loadb) nb = fetch<WM, 1>(g.Wt, g.sWn, g.sWk, n0, (t - t1) * BK, g.N, g.K2, tid);
+        }
+    };
+    auto put = [&](int t, int buf) {
+        if (t < t1) {
+            pair_park_a<WR, FM>(As[buf], na);
+            if (loadb) park<STAGE_MN>(Bs[buf], nb, tid);
+        } else {
+            pair_park_a<WR, STAGE_K>(As[buf], na);
+            if (loadb) park<WM>(Bs[buf], nb, tid);
+        }
+    };
+    get(0);
+    put(0, 0);
+    __syncthreads();
+    for (int t = 0; t < tiles; ++t) {
+        if (t + 1 < tiles) get(t + 1);
+        const int cur = t & 1, kq = (lane >> 4) * 8;
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[cur][wm + bi * 16 + (lane & 15)][kq]);
+#pragma unroll
+            for (int bj = 0; bj < 2; ++bj) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&Bs[cur][wn + bj * 16 + (lane & 15)][kq]);
+                if (t < t1) accF[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, accF[bi][bj], 0, 0, 0);
+                else accV[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, accV[bi][bj], 0, 0, 0);
+            }
+        }
+        if (t + 1 < tiles) put(t + 1, cur ^ 1);
+        __syncthreads();
+    }
+    const int mr = m0 + wm + (lane & 15), nc = n0 + wn + (lane >> 4) * 4;
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj) {
+            const int m = mr + bi * 16, n = nc + bj * 16;
+            if (m >= g.M || n >= g.N) continue;
+            const long o = ((long)z * g.M + m) * g.N + n;
+            f32x4 v = accV[bi][bj];
+            if (BWD) {
+                v = accF[bi][bj] + v;
+                *reinterpret_cast<f32x4 *>(g.y + o) = v;
+                continue;
+            }
+            v = v + *reinterpret_cast<const f32x4 *>(g.bias + n);
+            v = v + accF[bi][bj];
+            if (g.pre) *reinterpret_cast<f32x4 *>(g.pre + o) = v;
+            if (g.act == CGFD_FNO_ACT_GELU) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = gelu(v[i]);
+            }
+            *reinterpret_cast<f32x4 *>(g.y + o) = v;
+            u16x4 e;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) e[i] = to_bf16(v[i]);
+            *reinterpret_cast<u16x4 *>(g.yb + o) = e;
+        }
+}
+
+// strips of 32 points per block: the fewest strips in all, then the largest blocks
+template <int BWD> void launch_pair(const PairArgs &g, int batch, hipStream_t s)
+{
+    const int strips = (g.M + 31) / 32;
+    int wr = 4;
+    for (int c = 3; c >= 2; --c)
+        if ((strips + c - 1) / c * c < (strips + wr - 1) / wr * wr) wr = c;
+    const dim3 grid((g.N + BN - 1) / BN, (strips + wr - 1) / wr, batch);
+    if (wr == 4) hipLaunchKernelGGL((layer_pair_kernel<4, BWD>), grid, dim3(512), 0, s, g);
+    else if (wr == 3) hipLaunchKernelGGL((layer_pair_kernel<3, BWD>), grid, dim3(384), 0, s, g);
+    else hipLaunchKernelGGL((layer_pair_kernel<2, BWD>), grid, dim3(256), 0, s, g);
+}
+
 // rows of x and gz that one partial weight-gradient product covers
 constexpr int WROWS = 256;
 
@@ -708,7 +850,7 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
     int rc = check_layer(B, H, W, C, m);
     if (rc) return rc;
     if (!L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wre || !L->wim || !L->w || !L->bias || !L->wr || !L->wb ||
-        !L->t1 || !L->x || !L->t2 || !L->t3 || !L->sp || !L->y || !L->yb)
+        !L->t1 || !L->x || !L->t2 || !L->t3 || !L->y || !L->yb)
         return CGFD_FNO_EINVAL;
     const hipStream_t s = (hipStream_t)stream;
     const long mC = (long)m * C, C2 = 2L * C;
@@ -727,6 +869,15 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
     // t3 [b][(h,ri)][(kw,c)]
     product_bf16({L->gi, 0, 4L * m, 1}, {L->t2, 4 * m * mC, 1, mC}, rows(L->t3, 2 * H * mC, mC), 2 * H, m * C, 4 * m, B,
                  s);
+    // both in one launch where whole groups of eight can be staged
+    if (m % 4 == 0 && vec4(L->bias, 0, 0, 4)) {
+        PairArgs g{(const unsigned short *)L->fi, (const unsigned short *)L->t3, (const unsigned short *)L->vb,
+                   (const unsigned short *)L->wb, 2 * m, 1, 2 * mC, C, (long)W * C, C, 1, C, W, C, 2 * m, C,
+                   L->gelu ? CGFD_FNO_ACT_GELU : CGFD_FNO_ACT_NONE, L->bias, L->y, L->pre, (unsigned short *)L->yb};
+        launch_pair<0>(g, B * H, s);
+        return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
+    }
+    if (!L->sp) return CGFD_FNO_EINVAL;
     rc = cgfd_fno_gemm_bf16(L->fi, 0, 2 * m, 1, L->t3, 2 * mC, C, 1, L->sp, (long)W * C, C, W, C, 2 * m, B * H, 0,
                             stream);
     if (rc) return rc;
@@ -762,6 +913,13 @@ extern "C" int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *L, void *stream
                        L->gwim, n4, C);
     product_bf16({L->gh, 0, 1, 2L * H}, {L->t2, 4 * m * mC, 1, mC}, rows(L->t3, 2 * H * mC, mC), 2 * H, m * C, 4 * m, B,
                  s);
+    if (W % 8 == 0) {
+        PairArgs g{(const unsigned short *)L->fw, (const unsigned short *)L->t3, (const unsigned short *)L->gzb,
+                   (const unsigned short *)L->wb, 1, W, 2 * mC, C, (long)W * C, C, C, 1, W, C, 2 * m, C,
+                   CGFD_FNO_ACT_NONE, nullptr, L->gv, nullptr, nullptr};
+        launch_pair<1>(g, B * H, s);
+        return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
+    }
     rc = cgfd_fno_gemm_bf16(L->fw, 0, 1, W, L->t3, 2 * mC, C, 1, L->gv, (long)W * C, C, W, C, 2 * m, B * H, 0, stream);
     if (rc) return rc;
     return cgfd_fno_gemm_bf16(L->gzb, 0, C, 1, L->wb, 0, 1, C, L->gv, 0, C, (int)R, C, C, 1, 1, stream);

@@ -332,7 +332,8 @@ class _FourierLayer(torch.autograd.Function):
         new = lambda *n, dtype=torch.bfloat16: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
         wr, wb, x = new(P, 2 * C, 2 * C), new(C, C), new(P, B, 2 * C)
         t1, t2, t3 = new(2 * B * H * m * C), new(4 * B * m * m * C), new(2 * B * H * m * C)
-        sp, y, yb = new(v.shape, dtype=torch.float32), new(v.shape, dtype=torch.float32), new(v.shape)
+        y, yb = new(v.shape, dtype=torch.float32), new(v.shape)
+        sp = new(v.shape, dtype=torch.float32) if m % 4 or b.data_ptr() % 16 else None
         pre = new(v.shape, dtype=torch.float32) if gelu and keep else None
         arg = _Forward(B, H, W, C, m, int(gelu), _ptr(vb), *(_ptr(t) for t in mats), _ptr(wre), _ptr(wim), _ptr(w),
                        _ptr(b), _ptr(wr), _ptr(wb), _ptr(x), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(sp), _ptr(y), _ptr(pre),

@@ -63,7 +63,7 @@ typedef struct cgfd_fno_fourier {
     void *wr, *wb;                   /* written: the weights in bf16 [P, 2C, 2C], [C, C] */
     void *x;                         /* written: the kept modes in bf16 [P, B, 2C] */
     void *t1, *t2, *t3;              /* scratch, bf16: 2*B*H*m*C, 4*B*m*m*C, 2*B*H*m*C */
-    float *sp;                       /* scratch [R, C] */
+    float *sp;                       /* scratch [R, C]; may be null if modes % 4 == 0 */
     float *y, *pre;                  /* the result and (or null) the value before the GELU */
     void *yb;                        /* the result in bf16 */
 } cgfd_fno_fourier;

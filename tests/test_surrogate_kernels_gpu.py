@@ -120,7 +120,11 @@ def _parts_backward(ctx, gy, *unused):
 # rows of the transforms that are no multiple of 8, the smallest width, one
 # mode, a last layer without GELU (layers = 1) and one with it
 @pytest.mark.parametrize("B,H,W,C,m,layers", [(1, 4, 4, 8, 1, 1), (2, 9, 11, 8, 3, 2), (3, 16, 20, 24, 5, 2), (2, 33, 40, 64, 16, 1),
-                                              (5, 12, 26, 40, 6, 3)])
+                                              (5, 12, 26, 40, 6, 3),
+                                              # the last step in one launch both ways (2, 3 and 4 strips of 32 points, two
+                                              # blocks per row, two channel tiles), one way, the other way
+                                              (2, 16, 48, 8, 8, 2), (2, 8, 80, 72, 4, 2), (1, 9, 200, 8, 4, 2),
+                                              (1, 8, 128, 64, 4, 2), (1, 8, 100, 16, 4, 2), (1, 10, 72, 16, 5, 2)])
 def test_fourier_layer_against_single_products(B, H, W, C, m, layers, monkeypatch):
     net = surrogate.FNO2d(surrogate.NCH, 3, C, m, layers, proj=32, seed=3).cuda()
     assert surrogate.fused_layer_ok(B, H, W, C, m)
