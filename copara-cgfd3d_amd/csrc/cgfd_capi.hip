@@ -213,26 +213,31 @@ static void fb_signs(int t, int k, int *sx, int *sz)
     *sz = (((p == 1 || p == 2) ? 1 : 0) ^ (k & 1)) ? -1 : 1;
 }
 
+constexpr int kFewBlocks = 512; // two workgroups per CU
+
+// tiles of one z plane at tile width tw
+static long plane_tiles(const cgfd_ctx *c, int tw)
+{
+    const int tr = stage_tile_rows(tw);
+    return (long)((c->g.ni + tw - 1) / tw) * ((c->g.nj + tr - 1) / tr);
+}
+
 // Tile width of the default stage kernel: the one set or tuned, else 32 when a
 // row of ni cells takes over 8 % more lanes in 64-column tiles than in
 // 32-column ones.  Measured per stage: 80 cells (128 vs 96 lanes) 13 % and
 // 200 cells (256 vs 224) 10 % faster at 32; 600 cells (640 vs 608) 0.5 %
 // and 64 or 192 cells (no idle lanes) 1-16 % slower, so a 32 x 8 tile costs
-// about 6 % more per lane than a 64 x 4 one.  FP64 runs 64.
+// about 6 % more per lane than a 64 x 4 one.  In FP64, whose kernel is bound by
+// instructions at 2 wavefronts per SIMD, idle lanes cost in full: 160x144x96
+// 295 us at 64 (192 lanes), 244 at 32 (160).  A grid too small to fill the chip
+// gains nothing from fewer lanes and keeps 64 there.
 static bool narrow_pays(long lanes64, long lanes32) { return lanes64 * 100 > lanes32 * 108; }
 static int tile_width(const cgfd_ctx *c)
 {
-    if (c->prec == CGFD_FP64) return 64;
     if (c->tile_w) return c->tile_w;
     if (c->tile_pref) return c->tile_pref;
+    if (c->prec == CGFD_FP64 && 2 * plane_tiles(c, 64) * c->g.nk <= kFewBlocks) return 64;
     return narrow_pays((c->g.ni + 63) / 64 * 64, (c->g.ni + 31) / 32 * 32) ? 32 : 64;
-}
-
-// tiles of one z plane at tile width tw
-static long plane_tiles(const cgfd_ctx *c, int tw)
-{
-    const int tr = stage_tile_rows(c->prec == CGFD_FP64, tw);
-    return (long)((c->g.ni + tw - 1) / tw) * ((c->g.nj + tr - 1) / tr);
 }
 
 // z chunks per column sweep: about 2048 tiles in the launch (4096 workgroups,
@@ -244,7 +249,7 @@ static long plane_tiles(const cgfd_ctx *c, int tw)
 // A grid that has at most 2 workgroups per CU with 1 plane each takes 1
 // (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
 // 31.2 us at 1 plane, 29.3 at 2).
-constexpr int kChunkPlanes = 9, kFewBlocks = 512;
+constexpr int kChunkPlanes = 9;
 static void default_tuning(cgfd_ctx *c)
 {
     c->rows = 4;

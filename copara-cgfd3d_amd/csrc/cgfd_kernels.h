@@ -95,8 +95,8 @@ void launch_stage(int variant, int sx, int sz, int st, const StageArgs<R> &a, co
 // nblocks); all grids share the step phase and the metric mode hmet.
 // nctx = -n: n grids of one size and z-chunk length on one medium, the n
 // copies of each tile run one after another on one XCD (starts unused).
-// rows of a default stage-kernel tile of tw columns (64 or 32; FP64 runs 64)
-int stage_tile_rows(bool fp64, int tw);
+// rows of a default stage-kernel tile of tw columns (64 or 32)
+int stage_tile_rows(int tw);
 template <typename R>
 void launch_stage_batch(int sx, int sz, int st, int hmet, int hybrid, int tw, const StageArgs<R> *pa,
                         const int *starts, int nctx, int nblocks, int tinc, hipStream_t s);

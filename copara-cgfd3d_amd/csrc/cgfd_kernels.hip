@@ -2059,22 +2059,17 @@ __global__ void snap_kernel(const R *fw, long fs, const long *lin, int npts, int
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// The half-system kernel at the tile width a.tile (32 or 64 columns; FP64 always 64).
+// The half-system kernel at the tile width a.tile (32 or 64 columns).
 template <typename R, int SX, int SZ, int ST, int HM>
 static void launch_half(const StageArgs<R> &a, const StageArgs<R> *pa, const int *starts, int nctx, int nblocks,
                         int zchunks, hipStream_t s)
 {
-    const int tw = sizeof(R) == 4 ? a.tile : 64, tr = stage_tile_rows(sizeof(R) == 8, tw);
+    const int tw = a.tile, tr = stage_tile_rows(tw);
     const int ntx = (a.g.ni + tw - 1) / tw, nty = (a.g.nj + tr - 1) / tr;
     // two workgroups per tile, one per half of the system
     const dim3 grid(2u * (unsigned)(nblocks > 0 ? nblocks : ntx * nty * zchunks)), block(64, HALF_TY);
-    if constexpr (sizeof(R) == 4) {
-        if (tw == 32) {
-            stage_half_kernel<R, SX, SZ, ST, HM, 32><<<grid, block, 0, s>>>(pa, starts, nctx);
-            return;
-        }
-    }
-    stage_half_kernel<R, SX, SZ, ST, HM, 64><<<grid, block, 0, s>>>(pa, starts, nctx);
+    if (tw == 32) stage_half_kernel<R, SX, SZ, ST, HM, 32><<<grid, block, 0, s>>>(pa, starts, nctx);
+    else stage_half_kernel<R, SX, SZ, ST, HM, 64><<<grid, block, 0, s>>>(pa, starts, nctx);
 }
 
 template <typename R, int SX, int SZ, int ST>
@@ -2263,7 +2258,7 @@ __global__ void step_advance_kernel(int *step)
 
 void launch_step_advance(int *step, hipStream_t s) { step_advance_kernel<<<1, 64, 0, s>>>(step); }
 
-int stage_tile_rows(bool fp64, int tw) { return HALF_TY * (!fp64 && tw == 32 ? 2 : 1); }
+int stage_tile_rows(int tw) { return HALF_TY * (tw == 32 ? 2 : 1); }
 
 // batched trace gathers: blockIdx.y = grid, whose RecArgs block is
 // kCtxArgBytes from the previous grid's

@@ -1,0 +1,64 @@
+"""The stage kernel's half-system workgroups where they can go wrong: ragged
+tiles of either width and precision, z chunks of one plane, launches whose
+workgroups fill the XCD order partly, absorbing sides of different depth or
+none, against the CPU oracle value for value."""
+import numpy as np
+import pytest
+
+import cgfd3d
+import oracle
+import scenario
+from conftest import assert_same
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(sc, steps, prec, zchunks=0, conindex=None):
+    g = cgfd3d.Simulation(sc["ni"], sc["nj"], sc["nk"], sc["dh"], sc["dt"], sc["nt"],
+                          precision=cgfd3d.FP64 if prec == 64 else cgfd3d.FP32)
+    o = oracle.Oracle(sc["ni"], sc["nj"], sc["nk"], sc["dh"], sc["dt"], sc["nt"], double=prec == 64)
+    if conindex:
+        sc = dict(sc, conindex=conindex)
+    for e in (g, o):
+        e.setup(sc)
+    if zchunks:
+        g.set_tuning(zchunks)
+    rng = np.random.default_rng(5)
+    for c, a in enumerate(scenario.random_state((sc["ni"] + 6, sc["nj"] + 6, sc["nk"] + 6), rng)):
+        g.set_field(c, a)
+        o.set_field(c, a)
+    for e in (g, o):
+        e.run(steps)
+    for c in range(9):
+        assert_same(g.get_field(c), o.get_field(c), f"FW[{c}]")
+        for axis in range(3):
+            if g.aux_size(axis):
+                assert_same(g.get_aux(axis, c), o.get_aux(axis, c), f"FA{axis}[{c}]")
+    assert_same(g.get_seismo(), o.get_seismo(), "seismograms")
+    assert_same(g.get_pgv(), o.get_pgv(), "PGV")
+    width = g.tile_width()
+    g.close()
+    return width
+
+
+# columns one short of, at and one past a tile; rows past one and several rounds
+# of the 8 XCDs; layers on one side only, of different depth, on no side
+@pytest.mark.parametrize("ni,nj,nk,nabs", [(31, 37, 9, [3, 5, 2, 6, 3, 0]), (65, 18, 12, [0, 7, 4, 0, 2, 0]),
+                                           (96, 70, 7, [9, 2, 0, 5, 0, 0]), (129, 9, 11, [0, 0, 0, 0, 4, 0])])
+@pytest.mark.parametrize("prec", [32, 64])
+@pytest.mark.parametrize("shear", [True, False])
+def test_ragged_grids(ni, nj, nk, nabs, prec, shear):
+    sc = scenario.config_random(ni, nj, nk, 4, nabs, seed=ni, shear=shear)
+    _compare(sc, 4, prec)
+
+
+@pytest.mark.parametrize("zchunks", [1, 12, 4])
+def test_chunk_lengths(zchunks):
+    _compare(scenario.config_random(40, 32, 12, 4, [5, 4, 4, 5, 5, 0], seed=8), 4, 32, zchunks)
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(80, 40, 20), (70, 57, 23)])
+@pytest.mark.parametrize("conindex", [None, 12])
+def test_fp64_in_narrow_tiles(ni, nj, nk, conindex):
+    sc = scenario.config_random(ni, nj, nk, 4, [5, 4, 4, 5, 5, 0], seed=nk, shear=conindex is None)
+    assert _compare(sc, 4, 64, conindex=conindex) == 32
