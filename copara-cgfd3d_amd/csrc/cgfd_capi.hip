@@ -1122,9 +1122,6 @@ template <typename R> static int run_stage(cgfd_ctx *c)
     }
     HIPCHK(c, hipGetLastError());
     if (k == 3) {
-        if (c->currT < c->d.nt && c->nrecv)
-            launch_record<R>((const R *)c->set_ptr(SET_FW), c->g.fs, c->rlin, c->nrecv, (R *)c->seis, c->d.nt,
-                             c->d_step, c->stream);
         // SWpick after the step (simulation.cc:312-315): every tinv steps.  The
         // kernel checks the step itself; a captured cycle launches it every step.
         for (auto &sn : c->snaps) {
@@ -1133,7 +1130,8 @@ template <typename R> static int run_stage(cgfd_ctx *c)
             launch_snap<R>((const R *)c->set_ptr(SET_FW), c->g.fs, sn.lin, sn.npts, sn.c0, sn.ncomp, (R *)sn.buf,
                            c->d_step, tinv, sn.ntime, c->stream);
         }
-        launch_step_advance(c->d_step, c->stream);
+        launch_step_end<R>((const R *)c->set_ptr(SET_FW), c->g.fs, c->rlin, c->nrecv, (R *)c->seis, c->d.nt, c->d_step,
+                           c->stream);
         HIPCHK(c, hipGetLastError());
         c->currT++;
         c->stage = 0;

@@ -119,13 +119,12 @@ template <typename R> void launch_media_prep(const Geom &g, R *med, hipStream_t 
 // Trace and snapshot gathers after a step read the step number from the
 // device counter, so a captured step graph replays at any step.
 template <typename R>
-void launch_record(const R *fw, long fs, const long *rlin, int nrecv, R *seis, int nt, const int *step,
-                   hipStream_t s);
-template <typename R>
 void launch_snap(const R *fw, long fs, const long *lin, int npts, int c0, int ncomp, R *buf, const int *step,
                  int tinv, int ntime, hipStream_t s);
-// step counter += 1 (one thread)
-void launch_step_advance(int *step, hipStream_t s);
+// after a step's other launches: its traces (nrecv may be 0; steps past nt
+// record nothing), then step counter += 1
+template <typename R>
+void launch_step_end(const R *fw, long fs, const long *rlin, int nrecv, R *seis, int nt, int *step, hipStream_t s);
 // The batched forms read the RecArgs blocks of nctx argument images from pa:
 // trace gathers of every grid (grids without receivers return at once), and
 // every grid's step counter += 1.

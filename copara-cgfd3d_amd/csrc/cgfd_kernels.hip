@@ -2045,9 +2045,30 @@ __global__ void record_kernel(const R *fw, long fs, const long *rlin, int nrecv,
 {
     const int t = *step;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nrecv * NF) return;
+    if (i >= nrecv * NF || t >= nt) return;
     const int r = i / NF, c = i % NF;
     seis[((long)c * nrecv + r) * nt + t] = fw[c * fs + rlin[r]];
+}
+
+// The last launch of a step: the receivers' traces and the step counter, which
+// every other launch of the step has read.  One workgroup, so that the counter
+// moves after all of it has read it; a launch and the gap before it less than a
+// gather and a one-lane increment (40x32x20: 74.5 -> 73.0 us per step, 64x64x64
+// replayed 155 -> 153).  Up to kRecordOne values: 400 receivers, 3780 values, were
+// slower in one workgroup (200x200x150: 1539 -> 1549 us per step).
+constexpr int kRecordOne = 1024;
+template <typename R>
+__global__ void __launch_bounds__(1024) record_advance_kernel(const R *fw, long fs, const long *rlin, int nrecv,
+                                                              R *seis, int nt, int *step)
+{
+    const int t = *step;
+    if (t < nt)
+        for (int i = threadIdx.x; i < nrecv * NF; i += blockDim.x) {
+            const int r = i / NF, c = i % NF;
+            seis[((long)c * nrecv + r) * nt + t] = fw[c * fs + rlin[r]];
+        }
+    __syncthreads();
+    if (threadIdx.x == 0) *step = t + 1;
 }
 
 // snapshots (SWpick, calculate.cu:2360-2444): after step t with t % tinv == 0,
@@ -2252,21 +2273,22 @@ void launch_snap(const R *fw, long fs, const long *lin, int npts, int c0, int nc
                                                                 ntime);
 }
 
-template <typename R>
-void launch_record(const R *fw, long fs, const long *rlin, int nrecv, R *seis, int nt, const int *step,
-                   hipStream_t s)
-{
-    if (nrecv <= 0) return;
-    const int n = nrecv * NF;
-    record_kernel<R><<<(n + 255) / 256, 256, 0, s>>>(fw, fs, rlin, nrecv, seis, nt, step);
-}
-
 __global__ void step_advance_kernel(int *step)
 {
     if (threadIdx.x == 0) step[0] += 1;
 }
 
-void launch_step_advance(int *step, hipStream_t s) { step_advance_kernel<<<1, 64, 0, s>>>(step); }
+template <typename R>
+void launch_step_end(const R *fw, long fs, const long *rlin, int nrecv, R *seis, int nt, int *step, hipStream_t s)
+{
+    const int n = nrecv * NF;
+    if (n <= kRecordOne) {
+        record_advance_kernel<R><<<1, n > 256 ? 1024 : (n > 64 ? 256 : 64), 0, s>>>(fw, fs, rlin, nrecv, seis, nt, step);
+        return;
+    }
+    record_kernel<R><<<(n + 255) / 256, 256, 0, s>>>(fw, fs, rlin, nrecv, seis, nt, step);
+    step_advance_kernel<<<1, 64, 0, s>>>(step);
+}
 
 int stage_tile_rows(int tw) { return HALF_TY * (tw == 32 ? 2 : 1); }
 
@@ -2320,7 +2342,7 @@ void launch_step_advance_batch(const char *pa, int nctx, hipStream_t s)
     template void launch_from_padded<R>(const R *, R *, const Geom &, hipStream_t);                          \
     template void launch_src_prep<R>(const Geom &, const R *, const R *, const int4 *, const R *, const R *,  \
                                      R *, int, R, hipStream_t);                                               \
-    template void launch_record<R>(const R *, long, const long *, int, R *, int, const int *, hipStream_t); \
+    template void launch_step_end<R>(const R *, long, const long *, int, R *, int, int *, hipStream_t);       \
     template void launch_snap<R>(const R *, long, const long *, int, int, int, R *, const int *, int, int,   \
                                  hipStream_t);                                                              \
     template void launch_media_prep<R>(const Geom &, R *, hipStream_t);

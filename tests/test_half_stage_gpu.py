@@ -62,3 +62,24 @@ def test_chunk_lengths(zchunks):
 def test_fp64_in_narrow_tiles(ni, nj, nk, conindex):
     sc = scenario.config_random(ni, nj, nk, 4, [5, 4, 4, 5, 5, 0], seed=nk, shear=conindex is None)
     assert _compare(sc, 4, 64, conindex=conindex) == 32
+
+
+# values of one wavefront, one workgroup and past one workgroup's gather
+@pytest.mark.parametrize("nrecv", [0, 1, 7, 8, 113, 114])
+@pytest.mark.parametrize("graph", [False, True])
+def test_trace_gather_and_step_counter(nrecv, graph):
+    sc = scenario.config_random(24, 20, 10, 9, [3, 2, 2, 3, 2, 0], seed=3, nrecv=max(nrecv, 2))
+    sc["recv_locs"] = sc["recv_locs"][:nrecv]
+    g = cgfd3d.Simulation(sc["ni"], sc["nj"], sc["nk"], sc["dh"], sc["dt"], sc["nt"])
+    o = oracle.Oracle(sc["ni"], sc["nj"], sc["nk"], sc["dh"], sc["dt"], sc["nt"])
+    g.setup(sc)
+    o.setup(sc)
+    g.set_graph(graph)
+    g.run(9)
+    o.run(9)
+    assert g.step == 9
+    for c in range(9):
+        assert_same(g.get_field(c), o.get_field(c), f"FW[{c}]")
+    if nrecv:
+        assert_same(g.get_seismo(), o.get_seismo(), "seismograms")
+    g.close()
