@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[i] = gelu(v[i]);
                 }
-                *reinterpret_cast<f32x4 *>(C + m * g.sCm + n) = v;
+                if (g.C) *reinterpret_cast<f32x4 *>(C + m * g.sCm + n) = v;
                 if (Cb) {
                     u16x4 e;
 #pragma unroll
@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(128 * WR) layer_pair_kernel(PairArgs g)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] = gelu(v[i]);
             }
-            *reinterpret_cast<f32x4 *>(g.y + o) = v;
+            if (g.y) *reinterpret_cast<f32x4 *>(g.y + o) = v;
             u16x4 e;
 #pragma unroll
             for (int i = 0; i < 4; ++i) e[i] = to_bf16(v[i]);
@@ -850,7 +850,7 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
     int rc = check_layer(B, H, W, C, m);
     if (rc) return rc;
     if (!L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wre || !L->wim || !L->w || !L->bias || !L->wr || !L->wb ||
-        !L->t1 || !L->x || !L->t2 || !L->t3 || !L->y || !L->yb)
+        !L->t1 || !L->x || !L->t2 || !L->t3 || !L->yb)
         return CGFD_FNO_EINVAL;
     const hipStream_t s = (hipStream_t)stream;
     const long mC = (long)m * C, C2 = 2L * C;
@@ -877,7 +877,7 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
         launch_pair<0>(g, B * H, s);
         return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
     }
-    if (!L->sp) return CGFD_FNO_EINVAL;
+    if (!L->sp || !L->y) return CGFD_FNO_EINVAL;
     rc = cgfd_fno_gemm_bf16(L->fi, 0, 2 * m, 1, L->t3, 2 * mC, C, 1, L->sp, (long)W * C, C, W, C, 2 * m, B * H, 0,
                             stream);
     if (rc) return rc;
@@ -946,5 +946,36 @@ extern "C" int cgfd_fno_encode(const double *src, float *out, int n, int i0, int
     if (n == 0) return 0;
     hipLaunchKernelGGL(encode_kernel, dim3((wi * wj + 255) / 256, n), dim3(256), 0, (hipStream_t)stream, src, out, i0, j0,
                        wi, wj, dh, L);
+    return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
+}
+
+// y = act(x w + b) for the layers whose fp32 result nobody reads
+extern "C" int cgfd_fno_linear_fwd(const void *xb, const void *wb, const float *bias, float *pre, int act, void *yb,
+                                   long R, int K, int N, void *stream)
+{
+    if (!xb || !wb || !bias || !yb || R <= 0 || R > 0x7fffffffL || (R + BM - 1) / BM > 65535 || K <= 0 || N <= 0 ||
+        (act != CGFD_FNO_ACT_NONE && act != CGFD_FNO_ACT_GELU))
+        return CGFD_FNO_EINVAL;
+    GemmArgs g{};
+    g.A = (const unsigned short *)xb;
+    g.B = (const unsigned short *)wb;
+    g.sAm = K;
+    g.sAk = 1;
+    g.sBk = N;
+    g.sBn = 1;
+    g.sCm = N;
+    g.M = (int)R;
+    g.N = N;
+    g.K = K;
+    g.amode = stage_mode(xb, 0, K, 1);
+    g.bmode = stage_mode(wb, 0, 1, N);
+    g.bias = bias;
+    g.pre = pre;
+    g.act = act;
+    g.Cb = (unsigned short *)yb;
+    g.sEm = N;
+    g.vec = 1;
+    if (N % 4 != 0 || !vec4(bias, 0, 0, 4) || !vec4(pre, 0, N, 4) || !vec4(yb, 0, N, 2)) return CGFD_FNO_EINVAL;
+    launch_gemm(g, 1, (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
 }

@@ -66,9 +66,10 @@ def load_library():
         lib.cgfd_fno_adam.argtypes = [P, P, I, D, D, D, D, LL, I, P]
         lib.cgfd_fno_linear_bwd.argtypes = [P] * 11 + [L, I, I, P]
         lib.cgfd_fno_fourier_fwd.argtypes = lib.cgfd_fno_fourier_bwd.argtypes = [P, P]
+        lib.cgfd_fno_linear_fwd.argtypes = [P, P, P, P, I, P, L, I, I, P]
         lib.cgfd_fno_encode.argtypes = [P, P, I, I, I, I, I, D, D, P]
         for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam", "cgfd_fno_encode",
-                   "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd"):
+                   "cgfd_fno_linear_fwd", "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd"):
             getattr(lib, fn).restype = I
         _LIB = lib
     return _LIB
@@ -234,6 +235,35 @@ def _stream():
     return torch.cuda.current_stream().cuda_stream
 
 
+def _linear_grads(gy, pre, xb, wb, want_gx, gz=None):
+    """(gx or None, gw, gb) of y = act(x w + b) from contiguous fp32 gy, with
+    gy * GELU'(pre) into gz when given; wb at most 256 columns."""
+    (R, K), N, dev = xb.shape, wb.shape[1], gy.device
+    new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+    gzb, gx = new(R, N, dtype=torch.bfloat16), new(R, K) if want_gx else None
+    gw, gb, wpart, bpart = new(K, N), new(N), new(-(-R // WROWS) * K * N), new(-(-R // GROUP) * N)
+    rc = load_library().cgfd_fno_linear_bwd(_ptr(gy), _ptr(pre), _ptr(xb), _ptr(wb), _ptr(gz), _ptr(gzb), _ptr(wpart),
+                                            _ptr(bpart), _ptr(gx), _ptr(gw), _ptr(gb), R, K, N, _stream())
+    if rc != 0:
+        raise SurrogateError(f"cgfd_fno_linear_bwd returned {rc}")
+    return gx, gw, gb
+
+
+def _linear_bf16(xb, wb, b, gelu, keep):
+    """(act(x w + b) in bf16, the value before the GELU or None), without the
+    fp32 result.  The columns of wb are a multiple of 4."""
+    R, (K, N) = xb.shape[0], wb.shape
+    yb = torch.empty(R, N, device=xb.device, dtype=torch.bfloat16)
+    pre = torch.empty(R, N, device=xb.device) if gelu and keep else None
+    b = b.contiguous()
+    b = b.clone() if b.data_ptr() % 16 else b
+    rc = load_library().cgfd_fno_linear_fwd(_ptr(xb), _ptr(wb), _ptr(b), _ptr(pre), ACT_GELU if gelu else ACT_NONE,
+                                            _ptr(yb), R, K, N, _stream())
+    if rc != 0:
+        raise SurrogateError(f"cgfd_fno_linear_fwd returned {rc}")
+    return yb, pre
+
+
 class _Linear(torch.autograd.Function):
     """y = act(x @ w + b (+ d)) with x [R, K], w [K, N], b [N] and an
     optional residual d [R, N]: one product with the bias, the residual and
@@ -267,18 +297,11 @@ class _Linear(torch.autograd.Function):
     def backward(ctx, gy, *unused):
         xb, wb, pre = ctx.saved_tensors
         gy = gy.contiguous()
-        (R, K), N, dev = xb.shape, wb.shape[1], gy.device
+        R, N, dev = xb.shape[0], wb.shape[1], gy.device
         if N > 256 or not gy.is_cuda or gy.dtype != torch.float32:
             return _Linear._backward_parts(ctx, gy, xb, wb, pre)
-        new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
-        gz = new(R, N) if ctx.has_d and ctx.gelu else None
-        gzb, gx = new(R, N, dtype=torch.bfloat16), new(R, K) if ctx.needs_input_grad[0] else None
-        gw, gb, wpart, bpart = new(K, N), new(N), new(-(-R // WROWS) * K * N), new(-(-R // GROUP) * N)
-        rc = load_library().cgfd_fno_linear_bwd(_ptr(gy), _ptr(pre), _ptr(xb), _ptr(wb), _ptr(gz), _ptr(gzb),
-                                                _ptr(wpart), _ptr(bpart), _ptr(gx), _ptr(gw), _ptr(gb), R, K, N,
-                                                _stream())
-        if rc != 0:
-            raise SurrogateError(f"cgfd_fno_linear_bwd returned {rc}")
+        gz = torch.empty(R, N, device=dev) if ctx.has_d and ctx.gelu else None
+        gx, gw, gb = _linear_grads(gy, pre, xb, wb, ctx.needs_input_grad[0], gz)
         gd = (gz if ctx.gelu else gy) if ctx.has_d else None
         return None if gx is None else gx[:, :ctx.k], gw[:ctx.k], gb, gd, None, None, None, None
 
@@ -315,60 +338,135 @@ def fused_layer_ok(B, H, W, C, m):
             and (B * H * W + 63) // 64 <= 65535)
 
 
-class _FourierLayer(torch.autograd.Function):
-    """y = act(v w + b + K v), one Fourier layer, on the native launches of
-    cgfd_fno_fourier_fwd / _bwd: what _LeftConst, _Bmm and _Linear compute one
-    after another, with the intermediates in bf16 only and no permuted copies.
-    v [R, C] with its bf16 copy vb; returns y and its bf16 copy."""
+def _fourier_fwd(vb, wre, wim, w, b, dims, gelu, keep, want_y):
+    """One Fourier layer from v in bf16: (y or None, y in bf16, what its
+    backward needs).  y is made in any case where the native layer cannot do
+    without it."""
+    B, H, W, C, m = dims
+    R, P, dev = B * H * W, 2 * m * m, vb.device
+    wre, wim, w, b = (t.contiguous() for t in (wre, wim, w, b))
+    b = b.clone() if b.data_ptr() % 16 else b
+    new = lambda *n, dtype=torch.bfloat16: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+    wr, wb, x = new(P, 2 * C, 2 * C), new(C, C), new(P, B, 2 * C)
+    t1, t2, t3 = new(2 * B * H * m * C), new(4 * B * m * m * C), new(2 * B * H * m * C)
+    sp = new(R, C, dtype=torch.float32) if m % 4 else None
+    y = new(R, C, dtype=torch.float32) if want_y or m % 4 else None
+    yb, pre = new(R, C), new(R, C, dtype=torch.float32) if gelu and keep else None
+    arg = _Forward(B, H, W, C, m, int(gelu), _ptr(vb), *(_ptr(t) for t in dft_matrices(H, W, m, dev)), _ptr(wre),
+                   _ptr(wim), _ptr(w), _ptr(b), _ptr(wr), _ptr(wb), _ptr(x), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(sp),
+                   _ptr(y), _ptr(pre), _ptr(yb))
+    rc = load_library().cgfd_fno_fourier_fwd(ctypes.byref(arg), _stream())
+    if rc != 0:
+        raise SurrogateError(f"cgfd_fno_fourier_fwd returned {rc}")
+    return y, yb, (vb, wr, wb, x, pre)
+
+
+def _fourier_bwd(gy, kept, dims):
+    """(gv, gwre, gwim, gw, gb) from contiguous fp32 gy."""
+    vb, wr, wb, x, pre = kept
+    B, H, W, C, m = dims
+    R, P, dev, bf = B * H * W, 2 * m * m, gy.device, torch.bfloat16
+    new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
+    gzb, g = new(R, C, dtype=bf), new(P, B, 2 * C, dtype=bf)
+    t1, t2, t3 = new(2 * B * H * m * C, dtype=bf), new(4 * B * m * m * C, dtype=bf), new(2 * B * H * m * C, dtype=bf)
+    gwr, wpart, bpart = new(P, 2 * C, 2 * C), new(-(-R // WROWS) * C * C), new(-(-R // GROUP) * C)
+    gv, gwre, gwim, gw, gb = new(R, C), new(P, C, C), new(P, C, C), new(C, C), new(C)
+    arg = _Backward(B, H, W, C, m, 0, _ptr(gy), _ptr(pre), _ptr(vb), *(_ptr(t) for t in dft_matrices(H, W, m, dev)),
+                    _ptr(wr), _ptr(wb), _ptr(x), _ptr(gzb), _ptr(g), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(gwr),
+                    _ptr(wpart), _ptr(bpart), _ptr(gv), _ptr(gwre), _ptr(gwim), _ptr(gw), _ptr(gb))
+    rc = load_library().cgfd_fno_fourier_bwd(ctypes.byref(arg), _stream())
+    if rc != 0:
+        raise SurrogateError(f"cgfd_fno_fourier_bwd returned {rc}")
+    return gv, gwre, gwim, gw, gb
+
+
+def _native(x, *params):
+    """Whether the addresses of these (tensor, shape) pairs can be handed to
+    the native launches beside x: fp32 of that shape on x's device.  What is
+    not takes the general path, which converts or refuses it."""
+    return x.is_cuda and all(p.dtype == torch.float32 and p.device == x.device and tuple(p.shape) == shape
+                             for p, shape in params)
+
+
+def _aligned(gy):
+    gy = gy.contiguous()
+    return gy.clone() if gy.data_ptr() % 16 else gy
+
+
+class _Trunk(torch.autograd.Function):
+    """The lifting and all Fourier layers, x [R, cin] -> (v [R, C], its bf16
+    copy): what _Linear, _LeftConst and _Bmm compute one after another, on the
+    native launches.  Between the layers only the bf16 copy exists, the operand
+    of the next products: the fp32 value in between had no other reader, and
+    writing it was a third of a forward layer's last launch (48 maps of 80 x 80
+    at width 64, forward alone: 2.28 -> 2.11 ms; a training step of 32: 1.41 ->
+    1.35 ms, with the head's hidden layer in bf16 only as well).  The backward
+    ends at the lowest layer that has a gradient to deliver.
+    params: lift_w, lift_b, then spec_re, spec_im, pw_w, pw_b of every layer."""
 
     @staticmethod
-    def forward(ctx, v, vb, wre, wim, w, b, shape, m, gelu, keep):
-        B, H, W = shape
-        C, dev = v.shape[1], v.device
-        P = 2 * m * m
-        vb = (v.to(torch.bfloat16) if vb is None else vb).contiguous()
-        mats = dft_matrices(H, W, m, dev)
-        wre, wim, w, b = (t.contiguous() for t in (wre, wim, w, b))
-        new = lambda *n, dtype=torch.bfloat16: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
-        wr, wb, x = new(P, 2 * C, 2 * C), new(C, C), new(P, B, 2 * C)
-        t1, t2, t3 = new(2 * B * H * m * C), new(4 * B * m * m * C), new(2 * B * H * m * C)
-        y, yb = new(v.shape, dtype=torch.float32), new(v.shape)
-        sp = new(v.shape, dtype=torch.float32) if m % 4 or b.data_ptr() % 16 else None
-        pre = new(v.shape, dtype=torch.float32) if gelu and keep else None
-        arg = _Forward(B, H, W, C, m, int(gelu), _ptr(vb), *(_ptr(t) for t in mats), _ptr(wre), _ptr(wim), _ptr(w),
-                       _ptr(b), _ptr(wr), _ptr(wb), _ptr(x), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(sp), _ptr(y), _ptr(pre),
-                       _ptr(yb))
-        rc = load_library().cgfd_fno_fourier_fwd(ctypes.byref(arg), _stream())
-        if rc != 0:
-            raise SurrogateError(f"cgfd_fno_fourier_fwd returned {rc}")
+    def forward(ctx, x, dims, keep, *params):
+        K = x.shape[1]
+        pad = -K % 8
+        xb = _pad_cols(x.to(torch.bfloat16), pad).contiguous()
+        lw = _pad_rows(params[0].to(torch.bfloat16), pad).contiguous()
+        vb, _ = _linear_bf16(xb, lw, params[1], False, keep)
+        layers, y, saved = (len(params) - 2) // 4, None, [xb, lw]
+        for l in range(layers):
+            last = l == layers - 1
+            y, vb, kept = _fourier_fwd(vb, *params[2 + 4 * l:6 + 4 * l], dims, not last, keep, last)
+            saved += kept
         if keep:
-            ctx.save_for_backward(vb, wr, wb, x, pre, *mats)
-        ctx.dims = (B, H, W, C, m)
-        ctx.mark_non_differentiable(yb)
+            ctx.save_for_backward(*saved)
+        ctx.dims, ctx.k, ctx.layers = dims, K, layers
+        ctx.mark_non_differentiable(vb)
         ctx.set_materialize_grads(False)
-        return y, yb
+        return y, vb
 
     @staticmethod
     def backward(ctx, gy, *unused):
-        vb, wr, wb, x, pre, *mats = ctx.saved_tensors
-        B, H, W, C, m = ctx.dims
-        R, P, dev = B * H * W, 2 * m * m, gy.device
-        gy = gy.contiguous()
-        if gy.data_ptr() % 16:
-            gy = gy.clone()
-        new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
-        bf = torch.bfloat16
-        gzb, g = new(R, C, dtype=bf), new(P, B, 2 * C, dtype=bf)
-        t1, t2, t3 = new(2 * B * H * m * C, dtype=bf), new(4 * B * m * m * C, dtype=bf), new(2 * B * H * m * C, dtype=bf)
-        gwr, wpart, bpart = new(P, 2 * C, 2 * C), new(-(-R // WROWS) * C * C), new(-(-R // GROUP) * C)
-        gv, gwre, gwim, gw, gb = new(R, C), new(P, C, C), new(P, C, C), new(C, C), new(C)
-        arg = _Backward(B, H, W, C, m, 0, _ptr(gy), _ptr(pre), _ptr(vb), *(_ptr(t) for t in mats), _ptr(wr), _ptr(wb),
-                        _ptr(x), _ptr(gzb), _ptr(g), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(gwr), _ptr(wpart), _ptr(bpart),
-                        _ptr(gv), _ptr(gwre), _ptr(gwim), _ptr(gw), _ptr(gb))
-        rc = load_library().cgfd_fno_fourier_bwd(ctypes.byref(arg), _stream())
-        if rc != 0:
-            raise SurrogateError(f"cgfd_fno_fourier_bwd returned {rc}")
-        return gv, None, gwre, gwim, gw, gb, None, None, None, None
+        n, needs = 4 * ctx.layers, ctx.needs_input_grad
+        grads = [None] * n
+        if gy is None:
+            return (None,) * (5 + n)
+        saved, g = ctx.saved_tensors, _aligned(gy)
+        for l in reversed(range(ctx.layers)):
+            g, *grads[4 * l:4 * l + 4] = _fourier_bwd(g, saved[2 + 5 * l:7 + 5 * l], ctx.dims)
+            if not any(needs[:5 + 4 * l]):
+                return (None,) * 5 + tuple(grads)
+        gx, gw, gb = _linear_grads(g, None, saved[0], saved[1], needs[0])
+        return (None if gx is None else gx[:, :ctx.k], None, None, gw[:ctx.k], gb, *grads)
+
+
+class _Head(torch.autograd.Function):
+    """The two-layer projection v [R, C] -> [R, cout] with the hidden layer in
+    bf16 only."""
+
+    @staticmethod
+    def forward(ctx, v, vb, w1, b1, w2, b2, keep):
+        vb = (v.to(torch.bfloat16) if vb is None else vb).contiguous()
+        w1b, w2b = w1.to(torch.bfloat16).contiguous(), w2.to(torch.bfloat16).contiguous()
+        hb, pre = _linear_bf16(vb, w1b, b1, True, keep)
+        y = torch.empty(v.shape[0], w2.shape[1], device=v.device, dtype=torch.float32)
+        gemm(hb, w2b, y, bias=b2.contiguous())
+        if keep:
+            ctx.save_for_backward(vb, w1b, w2b, hb, pre)
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        vb, w1b, w2b, hb, pre = ctx.saved_tensors
+        needs = ctx.needs_input_grad
+        gh, gw2, gb2 = _linear_grads(gy.contiguous(), None, hb, w2b, any(needs[:4]))
+        if gh is None:
+            return None, None, None, None, gw2, gb2, None
+        gv, gw1, gb1 = _linear_grads(gh, pre, vb, w1b, needs[0])
+        return gv, None, gw1, gb1, gw2, gb2, None
+
+
+def fused_head_ok(C, hidden, cout):
+    """Whether _Head takes these widths (operands staged in whole groups)."""
+    return C % 8 == 0 and hidden % 8 == 0 and hidden <= 256 and cout <= 256
 
 
 class _Bmm(torch.autograd.Function):
@@ -621,13 +719,16 @@ class FNO2d(torch.nn.Module):
         every product's epilogue writes for the next products."""
         B, H, W, _ = x.shape
         R = B * H * W
+        C, P = self.width, 2 * self.modes * self.modes
+        per = [p for l in range(self.layers) for p in (self.spec_re[l], self.spec_im[l], self.pw_w[l], self.pw_b[l])]
+        if (backend == "mfma" and self.layers and R and fused_layer_ok(B, H, W, C, self.modes)
+                and _native(x, (self.lift_w, (x.shape[3], C)), (self.lift_b, (C,)),
+                            *zip(per, ((P, C, C), (P, C, C), (C, C), (C,)) * self.layers))):
+            v, vb = _Trunk.apply(x.reshape(R, -1), (B, H, W, self.width, self.modes), torch.is_grad_enabled(),
+                                 self.lift_w, self.lift_b, *per)
+            return v.reshape(B, H, W, self.width), vb
         v, vb = linear(x.reshape(R, -1), self.lift_w, self.lift_b, backend, want_bf16=True)
-        fused = backend == "mfma" and fused_layer_ok(B, H, W, self.width, self.modes)
         for l in range(self.layers):
-            if fused:
-                v, vb = _FourierLayer.apply(v, vb, self.spec_re[l], self.spec_im[l], self.pw_w[l], self.pw_b[l],
-                                            (B, H, W), self.modes, l < self.layers - 1, torch.is_grad_enabled())
-                continue
             sp = self._spectral(v.reshape(B, H, W, self.width), l, backend, vb).reshape(R, self.width)
             v, vb = linear(v, self.pw_w[l], self.pw_b[l], backend, d=sp, gelu=l < self.layers - 1, xb=vb,
                            want_bf16=True)
@@ -636,6 +737,13 @@ class FNO2d(torch.nn.Module):
     def head(self, v, backend="mfma", vb=None):
         """The two-layer projection of a latent to the output channels."""
         B, H, W, _ = v.shape
+        (C, hidden), cout = self.p1_w.shape, self.p2_w.shape[1]
+        if (backend == "mfma" and v.numel() and v.shape[3] == C and fused_head_ok(C, hidden, cout)
+                and (vb is None or vb.dtype == torch.bfloat16 and vb.device == v.device and vb.shape == (B * H * W, C))
+                and _native(v, (self.p1_w, (C, hidden)), (self.p1_b, (hidden,)), (self.p2_w, (hidden, cout)),
+                            (self.p2_b, (cout,)))):
+            return _Head.apply(v.reshape(B * H * W, self.width), vb, self.p1_w, self.p1_b, self.p2_w, self.p2_b,
+                               torch.is_grad_enabled()).reshape(B, H, W, -1)
         h, hb = linear(v.reshape(B * H * W, self.width), self.p1_w, self.p1_b, backend, gelu=True, xb=vb,
                        want_bf16=True)
         return linear(h, self.p2_w, self.p2_b, backend, xb=hb).reshape(B, H, W, -1)

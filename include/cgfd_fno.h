@@ -64,7 +64,7 @@ typedef struct cgfd_fno_fourier {
     void *x;                         /* written: the kept modes in bf16 [P, B, 2C] */
     void *t1, *t2, *t3;              /* scratch, bf16: 2*B*H*m*C, 4*B*m*m*C, 2*B*H*m*C */
     float *sp;                       /* scratch [R, C]; may be null if modes % 4 == 0 */
-    float *y, *pre;                  /* the result and (or null) the value before the GELU */
+    float *y, *pre;                  /* the result (or null if modes % 4 == 0) and the value before the GELU (or null) */
     void *yb;                        /* the result in bf16 */
 } cgfd_fno_fourier;
 int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *layer, void *stream);
@@ -83,6 +83,11 @@ typedef struct cgfd_fno_fourier_grad {
     float *gv, *gwre, *gwim, *gw, *gb;
 } cgfd_fno_fourier_grad;
 int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *layer, void *stream);
+
+/* yb = act(x w + bias) in bf16 only, x [R, K] and w [K, N] in bf16, N a multiple
+ * of 4; the value before the activation into pre unless null. */
+int cgfd_fno_linear_fwd(const void *xb, const void *wb, const float *bias, float *pre, int act, void *yb, long R,
+                        int K, int N, void *stream);
 
 /* Gradients of y = act(x w + b (+ d)) from gy [R, N], x [R, K] and w [K, N] in
  * bf16: gz = gy * GELU'(pre) (pre null: gy), in bf16 into gzb and on request

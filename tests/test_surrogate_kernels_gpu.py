@@ -133,6 +133,7 @@ def test_fourier_layer_against_single_products(B, H, W, C, m, layers, monkeypatc
     for fused in (True, False):
         if not fused:
             monkeypatch.setattr(surrogate, "fused_layer_ok", lambda *a: False)
+            monkeypatch.setattr(surrogate, "fused_head_ok", lambda *a: False)
         net.zero_grad(set_to_none=True)
         y = net(x)
         y.backward(gy)
@@ -149,6 +150,32 @@ def test_fourier_layer_against_single_products(B, H, W, C, m, layers, monkeypatc
         else:
             scale = float(g.abs().max()) + 1e-30
             assert float((g - got[1][1][n]).abs().max()) <= (B * H * W + 4) * EPS * scale, n
+
+
+# parameters that the native launches don't take go the general way: refused
+# there, or converted; frozen layers get no gradient and change no other
+def test_trunk_with_other_parameters():
+    net = surrogate.FNO2d(surrogate.NCH, 3, 16, 4, 3, proj=32, seed=3).cuda()
+    x = _rand((2, 12, 16, surrogate.NCH), 1).cuda()
+    y = net(x)
+    y.square().sum().backward()
+    want = {n: p.grad.clone() for n, p in net.named_parameters()}
+    net.zero_grad(set_to_none=True)
+    names = [n for n, _ in net.named_parameters()]
+    for frozen in (["lift_w", "lift_b", "spec_re.0", "spec_im.0", "pw_w.0", "pw_b.0"], ["p1_w", "p1_b"],
+                   [n for n in names if not n.startswith("p2")]):
+        for n, p in net.named_parameters():
+            p.requires_grad_(n not in frozen)
+        net(x).square().sum().backward()
+        for n, p in net.named_parameters():
+            assert (p.grad is None) if n in frozen else torch.equal(p.grad, want[n]), n
+        net.zero_grad(set_to_none=True)
+    with pytest.raises(surrogate.SurrogateError):
+        net(x[..., :-1].contiguous())
+    net.spec_re[1].data = net.spec_re[1].data.double()
+    assert torch.equal(net(x), y)
+    with pytest.raises(surrogate.SurrogateError):
+        net.double()(x)
 
 
 # operands staged whole (extents in multiples of 8), groups of eight that cross
