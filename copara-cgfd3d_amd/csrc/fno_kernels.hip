@@ -16,7 +16,7 @@
 // (v_mfma_f32_16x16x32_bf16, gfx950).
 #include <hip/hip_runtime.h>
 
-#include "cgfd_fno.h"
+#include "fno_network.h"
 
 namespace {
 
