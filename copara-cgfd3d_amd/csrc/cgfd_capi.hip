@@ -224,10 +224,11 @@ static long plane_tiles(const cgfd_ctx *c, int tw)
 
 // Tile width of the default stage kernel: the one set or tuned, else 32 when a
 // row of ni cells takes over 8 % more lanes in 64-column tiles than in
-// 32-column ones.  Measured per stage: 80 cells (128 vs 96 lanes) 13 % and
-// 200 cells (256 vs 224) 10 % faster at 32; 600 cells (640 vs 608) 0.5 %
-// and 64 or 192 cells (no idle lanes) 1-16 % slower, so a 32 x 8 tile costs
-// about 6 % more per lane than a 64 x 4 one.  In FP64, whose kernel is bound by
+// 32-column ones.  Measured per stage in FP32: 80 cells (128 vs 96 lanes) 36.7
+// us at 64 and 35.4 at 32, 160 (192 vs 160) 134 and 122, 200 (256 vs 224) 329
+// and 314; 600 (640 vs 608) 4.50 and 4.62 ms; without idle lanes 192 cells 158
+// and 164 us, 320 cells 737 and 763, 64 cells 26.1 and 26.6: a 32 x 8 tile costs
+// 2-4 % more per lane than a 64 x 4 one.  In FP64, whose kernel is bound by
 // instructions at 2 wavefronts per SIMD, idle lanes cost in full: 160x144x96
 // 295 us at 64 (192 lanes), 244 at 32 (160).  A grid too small to fill the chip
 // gains nothing from fewer lanes and keeps 64 there.
@@ -245,7 +246,7 @@ static int tile_width(const cgfd_ctx *c)
 // chunks keep the launch's tail short and neighbouring tiles, which share halo
 // lines, close in time; each costs its first window again (4 planes).
 // Measured at 9 / 15 / 30 planes: 200x200x150 357 / 382 / 423 us, 600x600x300
-// 4.78 / 4.81 / 4.87 ms, 32 grids of 80x80x48 per step 4.92 / 4.92 / 5.03 ms.
+// 4.78 / 4.81 / 4.87 ms, 32 grids of 80x80x48 per step 3.30 / 3.28 / 3.36 ms (at 9 / 15 / 25).
 // A grid that has at most 2 workgroups per CU with 1 plane each takes 1
 // (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
 // 31.2 us at 1 plane, 29.3 at 2).
@@ -913,11 +914,19 @@ int cgfd_init(cgfd_ctx *c)
     // FW and tW are what a caller can read before the first stage; the stage
     // outputs S1 and S2 are written in every valid cell before they are read,
     // and their guard cells, zero since the allocation, never get another value
-    // (600x600x300: 21 GB cleared in 5.2 ms, now half)
+    // (600x600x300: 21 GB cleared in 5.2 ms, now half).  Where all four are
+    // cleared in the time of the further calls, up to four of ~5 us at 6 TB/s,
+    // one call per array clears them together.
+    const size_t set_bytes = (size_t)NF * c->g.fs * c->esz;
+    const bool all = NSETS * set_bytes <= (size_t)128 << 20;
+    const size_t n = all ? NSETS : 1;
     for (int s : {SET_FW, SET_TW}) {
-        HIPCHK(c, hipMemsetAsync(c->set_ptr(s), 0, (size_t)NF * c->g.fs * c->esz, c->stream));
+        const int first = all ? 0 : s;
+        HIPCHK(c, hipMemsetAsync(c->set_ptr(first), 0, n * set_bytes, c->stream));
         for (int a = 0; a < 3; a++)
-            if (c->aux[a]) HIPCHK(c, hipMemsetAsync(c->aux_ptr(a, s), 0, (size_t)NF * c->astr[a] * c->esz, c->stream));
+            if (c->aux[a])
+                HIPCHK(c, hipMemsetAsync(c->aux_ptr(a, first), 0, n * NF * c->astr[a] * c->esz, c->stream));
+        if (all) break;
     }
     HIPCHK(c, hipMemsetAsync(c->pgv, 0, (size_t)3 * c->cstr * c->esz, c->stream));
     HIPCHK(c, hipMemsetAsync(c->timg, 0, (size_t)9 * c->tstr * c->esz, c->stream));

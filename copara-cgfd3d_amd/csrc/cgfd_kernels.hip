@@ -685,7 +685,9 @@ __global__ void __launch_bounds__(256) stage_direct_kernel(const StageArgs<R> *p
 // Stage kernel, one cell per lane -> two halves: 600x600x300 5.31 -> 5.15 ms,
 // 200x200x150 428 -> 411 us, 149x131x97 with all nine metrics 171 -> 150 us,
 // 160x144x96 FP64 415 -> 313 us, 64x64x64 31.3 -> 27.8 us, 40x32x20 20.5 ->
-// 15.4 us.  Measured and not taken: both halves in one workgroup of 8
+// 15.4 us.  With the x auxiliaries per side, the shorter chunks, the tile map
+// and the FP64 tile width they are at 4.75 ms, 352, 136, 244, 26.8 and 11.8 us.
+// Measured and not taken: both halves in one workgroup of 8
 // wavefronts that share the tile (5.24 ms, 160 us: each plane waits for the
 // slower half), the absorbing operands loaded ahead of the stencil (its
 // registers cost a wavefront per SIMD), the tiles of odd stages in reverse
