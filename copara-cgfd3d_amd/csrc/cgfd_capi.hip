@@ -992,6 +992,7 @@ template <typename R> static StageArgs<R> make_stage_args(const cgfd_ctx *c, int
     sa.med = (const R *)c->med;
     sa.pml = (const R *)c->pml;
     memcpy(sa.nabs, c->nabs, sizeof(sa.nabs));
+    sa.aux = aux_x_layout(c->nabs[0], c->nabs[1], c->g.ni, c->g.nj, c->g.nk);
     for (int a = 0; a < 3; a++) {
         sa.npml[a] = c->npml[a];
         sa.astr[a] = c->astr[a];
@@ -1037,6 +1038,7 @@ template <typename R> static TimgArgs<R> make_timg_args(const cgfd_ctx *c, int k
     ta.med = (const R *)c->med;
     ta.pml = (const R *)c->pml;
     memcpy(ta.nabs, c->nabs, sizeof(ta.nabs));
+    ta.aux = aux_x_layout(c->nabs[0], c->nabs[1], c->g.ni, c->g.nj, c->g.nk);
     for (int a = 0; a < 2; a++) {
         ta.npml[a] = c->npml[a];
         ta.astr[a] = c->astr[a];
@@ -1700,7 +1702,7 @@ static long aux_engine_index(const cgfd_ctx *c, int axis, int pidx, int a, int b
 {
     // axis 0: (px, y, z); axis 1: (py, x, z); axis 2: (pz, x, y), all 0-based valid
     if (axis == 0) // the reference's packed index counts the low side's layers, then the high side's
-        return aux_x_index(c->nabs[0], c->nabs[1], c->g.ni, c->g.nj, c->g.nk,
+        return aux_x_index(aux_x_layout(c->nabs[0], c->nabs[1], c->g.ni, c->g.nj, c->g.nk), c->nabs[0], c->g.nj,
                            pidx < c->nabs[0] ? pidx : c->g.ni - c->npml[0] + pidx, a, b);
     if (axis == 1) return ((long)b * c->npml[1] + pidx) * c->g.nxp + a;
     return ((long)pidx * c->g.nj + b) * c->g.nxp + a;

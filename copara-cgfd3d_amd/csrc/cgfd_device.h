@@ -47,17 +47,33 @@ __device__ __forceinline__ long gidx(const Geom &g, int x, int y, int z)
     return g.base + ((long)z * g.nyp + y) * g.nxp + x;
 }
 
-// Element of cell (x, y, z) in an x-axis auxiliary field: the n0 layers of the
-// low side as [z][y][n0], then the n1 of the high side as [z][y][n1].  A tile
-// touches one side only; with both sides in one row its few cells per row
-// would lie n0 + n1 apart, and every row would fetch cache lines that belong
-// mostly to the other side (80-cell rows with 10 + 10 layers: four times the
-// bytes used).
-// A padded field is below 4 GiB, so 32 bits hold the element.
-__host__ __device__ inline unsigned aux_x_index(int n0, int n1, int ni, int nj, int nk, int x, int y, int z)
+// Element of cell (x, y, z) in an x-axis auxiliary field, laid out so that what
+// one tile touches of a row lies together.  Rows of more than one tile: the n0
+// layers of the low side as [z][y][n0], then the n1 of the high side as
+// [z][y][n1], since a tile touches one side only; with both sides in one row its
+// few cells per row would lie n0 + n1 apart, and every row would fetch cache
+// lines that belong mostly to the other side (80-cell rows with 10 + 10 layers:
+// four times the bytes used).  Rows of one 64-column tile: [z][y][n0 + n1], since
+// the tile touches both sides; in two blocks each would be half as long and
+// twice as many lines would be shared with the rows of other tiles (stage and
+// traction image of 20 grids of 60x60x60 on one medium 377 -> 325 us, of 32 of
+// 40x40x32 234 -> 206, of 20 of 64x64x64 387 -> 344; one 64x64x64 31.0 -> 29.5).
+// A padded field is below 4 GiB, so 32 bits hold the element.  The strides are
+// formed once on the host: selecting them per cell cost small grids 2-3 %.
+struct AuxX {
+    unsigned len0, len1; // elements per row of the low and of the high side's block
+    unsigned shift;      // where the high side begins, less its first column (modulo 2^32)
+};
+__host__ __device__ inline AuxX aux_x_layout(int n0, int n1, int ni, int nj, int nk)
+{
+    const bool one = ni <= 64;
+    const unsigned high = one ? n0 : (unsigned)nk * nj * n0;
+    return {(unsigned)(one ? n0 + n1 : n0), (unsigned)(one ? n0 + n1 : n1), high - (unsigned)(ni - n1)};
+}
+__host__ __device__ inline unsigned aux_x_index(AuxX ax, int n0, int nj, int x, int y, int z)
 {
     const unsigned row = (unsigned)z * nj + y;
-    return x < n0 ? row * n0 + x : (unsigned)nk * nj * n0 + row * n1 + (x - (ni - n1));
+    return x < n0 ? row * ax.len0 + x : row * ax.len1 + x + ax.shift;
 }
 
 // Correctly rounded s/h for a fixed divisor h, given rh = RN(1/h): one

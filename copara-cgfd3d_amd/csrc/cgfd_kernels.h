@@ -17,6 +17,7 @@ template <typename R> struct StageArgs {
     const R *med; // lam2mu, miu, 1/rho, rho at stride g.fs
     const R *pml; // APD B DB for x (ni each), then y (nj each), then z (nk each)
     int nabs[6];
+    AuxX aux;      // layout of the x-axis auxiliary fields
     int npml[3];   // packed PML widths per axis
     long astr[3];  // stride between the 9 components of one auxiliary set
     const R *ain[3];
@@ -53,6 +54,7 @@ template <typename R> struct TimgArgs {
     const R *med; // lam2mu, miu, 1/rho, rho
     const R *pml;
     int nabs[6];
+    AuxX aux;
     int npml[2];
     long astr[2];
     const R *ain[2];

@@ -118,6 +118,9 @@ template <typename AP> __device__ __forceinline__ Geom geom_of(AP a)
     return g;
 }
 
+// the same for the x-axis auxiliary layout
+template <typename AP> __device__ __forceinline__ AuxX aux_x_of(AP a) { return {a->aux.len0, a->aux.len1, a->aux.shift}; }
+
 // per-(x,y)-column constants of the PML and source bookkeeping
 template <typename R> struct Column {
     R APDx, Bx, DBx, APDy, By, DBy;
@@ -406,7 +409,7 @@ __device__ __forceinline__ void cell_rates(AP a, const Column<R> &k, const CellI
     }
     if (k.inx) {
         const R APDx = k.APDx, DBx = k.DBx;
-        const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
+        const long aidx = aux_x_index(aux_x_of(a), a->nabs[0], g.nj, x, y, z);
         AuxIn<R> v;
         load_aux<R, ST>(a, 0, aidx, v);
         R ha[NF];
@@ -950,7 +953,7 @@ __device__ __forceinline__ void half_rates(AP a, const HalfCol<R> &k, const Half
     const unsigned tcell = (unsigned)(top > 0 ? top : 0) * (unsigned)(g.nj * g.nxp) + cxy;
     if (k.inx) {
         const R APDx = k.APDx, DBx = k.DBx;
-        const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
+        const long aidx = aux_x_index(aux_x_of(a), a->nabs[0], g.nj, x, y, z);
         HalfAux<R, PART> v;
         load_half_aux<R, ST, PART>(a, 0, aidx, v);
         R ha[NO];
@@ -1590,7 +1593,7 @@ stage_split_kernel(const StageArgs<R> *pa, int tinc)
                 }
             };
             if (k.inx) {
-                const long aidx = aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z);
+                const long aidx = aux_x_index(aux_x_of(a), a->nabs[0], g.nj, x, y, z);
                 R ai[NO], ha[NO];
 #pragma unroll
                 for (int c = 0; c < NO; ++c) ai[c] = a->ain[0][(C0 + c) * a->astr[0] + aidx];
@@ -1852,7 +1855,7 @@ __global__ void __launch_bounds__(256) timg_kernel(const TimgArgs<R> av, const T
             const R DzTz = (R)((double)rhojac * (drp_sum_strf<R, SZ>(vz[m]) / hz));
             R hv = (Bx == (R)1 && By == (R)1) ? DxTx + DyTy + DzTz : DxTx / Bx + DyTy / By + DzTz;
             if (inx) {
-                const R av = a->ain[0][m * a->astr[0] + aux_x_index(a->nabs[0], a->nabs[1], g.ni, g.nj, g.nk, x, y, z)];
+                const R av = a->ain[0][m * a->astr[0] + aux_x_index(aux_x_of(a), a->nabs[0], g.nj, x, y, z)];
                 hv -= av / Bx;
                 a->timg[(3 + m) * a->tstr + tcell] = DBx * DxTx - APDx * av;
             }
