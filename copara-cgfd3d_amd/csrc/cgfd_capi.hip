@@ -250,17 +250,31 @@ static int tile_width(const cgfd_ctx *c)
 // A grid that has at most 2 workgroups per CU with 1 plane each takes 1
 // (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
 // 31.2 us at 1 plane, 29.3 at 2).
+// The FP32 kernel that loads all nine metrics holds 3 workgroups per CU (4 with
+// constant horizontal metrics): a launch of 2-plane chunks just past that takes
+// 3 planes if those fit at once (64x64x64 35.4 -> 32.3 us with the traction image,
+// 64x64x50 31.0 -> 29.8, 48x64x70 37.2 -> 32.4, 60x60x60 33.2 both ways).
 constexpr int kChunkPlanes = 9;
+constexpr int kNineMetricBlocks = 3 * 256;
+static int default_zchunks(const cgfd_ctx *c)
+{
+    const long tiles = plane_tiles(c, tile_width(c));
+    const int nk = c->g.nk;
+    auto blocks = [&](long zc) { return 2 * tiles * zc; };
+    long zc = std::max((2048 + tiles - 1) / tiles, (long)(nk + kChunkPlanes - 1) / kChunkPlanes);
+    const int least = blocks(nk) <= kFewBlocks ? 1 : 2; // planes of the shortest chunk
+    zc = std::max(1L, std::min(zc, (long)std::max(1, nk / least)));
+    const bool nine = c->prec == CGFD_FP32 && !(c->hmet && c->use_hmet);
+    if (nine && zc == nk / 2 && blocks(zc) > kNineMetricBlocks && blocks((nk + 2) / 3) <= kNineMetricBlocks)
+        zc = (nk + 2) / 3;
+    return (int)zc;
+}
 static void default_tuning(cgfd_ctx *c)
 {
     c->rows = 4;
-    const long tiles = plane_tiles(c, tile_width(c));
-    long zc = std::max((2048 + tiles - 1) / tiles, (long)(c->g.nk + kChunkPlanes - 1) / kChunkPlanes);
-    const int least = 2 * tiles * c->g.nk <= kFewBlocks ? 1 : 2; // planes of the shortest chunk
-    zc = std::max(1L, std::min(zc, (long)std::max(1, c->g.nk / least)));
-    c->zchunks = (int)zc;
-    c->zc_tuned = false;
     c->tile_pref = 0;
+    c->zchunks = default_zchunks(c);
+    c->zc_tuned = false;
 }
 
 extern "C" {
@@ -911,6 +925,10 @@ int cgfd_init(cgfd_ctx *c)
     if (!c) return CGFD_EINVAL;
     if (!c->have_metrics || !c->have_media) return fail(c, CGFD_ESTATE, "metrics and media must be set before init");
     HIPCHK(c, hipSetDevice(c->dev));
+    if (!c->zc_tuned && c->zchunks != default_zchunks(c)) { // the metrics decide which kernel runs
+        c->zchunks = default_zchunks(c);
+        c->args_dirty = true;
+    }
     // FW and tW are what a caller can read before the first stage; the stage
     // outputs S1 and S2 are written in every valid cell before they are read,
     // and their guard cells, zero since the allocation, never get another value

@@ -83,3 +83,17 @@ def test_trace_gather_and_step_counter(nrecv, graph):
     if nrecv:
         assert_same(g.get_seismo(), o.get_seismo(), "seismograms")
     g.close()
+
+
+# grids whose 2-plane chunks are just past what the chip holds of the kernel for
+# nine metrics, at it, and whose 3-plane chunks are past it too
+@pytest.mark.parametrize("ni,nj,nk,shear,chunks", [(64, 64, 64, True, 22), (64, 64, 48, True, 24), (60, 57, 60, True, 20),
+                                                   (64, 64, 96, True, 48), (64, 64, 64, False, 32)])
+def test_chunks_of_a_launch_just_past_one_round(ni, nj, nk, shear, chunks):
+    sc = scenario.config_random(ni, nj, nk, 1, [5, 4, 4, 5, 5, 0], seed=nk, shear=shear)
+    g = cgfd3d.Simulation(ni, nj, nk, sc["dh"], sc["dt"], 1)
+    g.setup(sc)
+    assert g.metrics_specialized() == (not shear)
+    assert g.autotune() == chunks  # with one step there is nothing to time: the default choice
+    g.close()
+    _compare(sc, 1, 32)
