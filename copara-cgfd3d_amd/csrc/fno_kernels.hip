@@ -436,25 +436,34 @@ __global__ void __launch_bounds__(256) layer_grad_kernel(const float *__restrict
 }
 
 // out[i] = sum over n of part[n][i] for the weight gradient (first blocks) and
-// the bias gradient, summed in double.  1024 lanes: 64 columns, 16 slices.
+// the bias gradient, summed in double.  1024 lanes: 1024/SL columns, each in SL
+// slices.  Many parts of few columns need the slices to fill the chip
+// (262144 x 64 x 64, 1024 parts, with the whole gradient: 62 us with 16 slices,
+// 188 with 1); with few parts most slices have none (1024 x 8192 x 256, 4 parts:
+// 120 us with 16, 75 with 1).
+template <int SL>
 __global__ void __launch_bounds__(1024) layer_reduce_kernel(const float *__restrict__ wpart, int nw, int W,
                                                             float *__restrict__ gw, const float *__restrict__ bpart,
                                                             int nb, int N, float *__restrict__ gb, int wblocks)
 {
-    __shared__ double acc[16][64];
+    constexpr int COLS = 1024 / SL;
+    __shared__ double acc[SL][COLS];
     const bool isw = (int)blockIdx.x < wblocks;
     const float *src = isw ? wpart : bpart;
     const int n = isw ? nw : nb, len = isw ? W : N;
-    const int c = (isw ? blockIdx.x : blockIdx.x - wblocks) * 64 + threadIdx.x % 64, sl = threadIdx.x / 64;
+    const int col = threadIdx.x % COLS, sl = threadIdx.x / COLS;
+    const int c = (isw ? blockIdx.x : blockIdx.x - wblocks) * COLS + col;
     double s = 0.0;
     if (c < len) {
 #pragma unroll 4
-        for (int k = sl; k < n; k += 16) s += (double)src[(long)k * len + c];
+        for (int k = sl; k < n; k += SL) s += (double)src[(long)k * len + c];
     }
-    acc[sl][threadIdx.x % 64] = s;
-    __syncthreads();
+    if (SL > 1) {
+        acc[sl][col] = s;
+        __syncthreads();
+    }
     if (sl == 0 && c < len) {
-        for (int k = 1; k < 16; ++k) s += acc[k][threadIdx.x];
+        for (int k = 1; k < SL; ++k) s += acc[k][col];
         (isw ? gw : gb)[c] = (float)s;
     }
 }
@@ -631,15 +640,25 @@ template <int BWD> void launch_pair(const PairArgs &g, int batch, hipStream_t s)
     else hipLaunchKernelGGL((layer_pair_kernel<2, BWD>), grid, dim3(256), 0, s, g);
 }
 
-// rows of x and gz that one partial weight-gradient product covers
-constexpr int WROWS = 256;
+// Rows of x and gz that one partial weight-gradient product covers: 256, or 512
+// for weights of at least 16 tiles where the parts then still are 8 blocks per CU.
+// 256 / 512 rows, gw and gb alone: 65536 x 256 x 256 123 / 115 us, 65536 x 2048 x 256
+// 655 / 606 (256 rows write twice the partial sums), 32768 x 64 x 64 22.5 / 28.7, 2048
+// x 512 x 256 41 / 46 (512 rows leave the chip idle); 300000 x 128 x 128 with its
+// forward pass 325 / 332 (the last part runs alone, for longer).
+int weight_rows(long R, int K, int N)
+{
+    const long tiles = (long)((K + BM - 1) / BM) * ((N + BN - 1) / BN);
+    return tiles >= 16 && R / 512 * tiles >= 2048 ? 512 : 256;
+}
 
 // Gradients of y = x w + b after its epilogue: gzb and (optional) gz from gy
-// and pre, gw and gb.  wpart: ceil(R/WROWS) x K x N, bpart: ceil(R/GROUP) x N.
+// and pre, gw and gb.  wpart: ceil(R/weight_rows) x K x N, bpart: ceil(R/GROUP) x N.
 void linear_grads(const float *gy, const float *pre, const void *xb, float *gz, void *gzb, float *wpart, float *bpart,
                   float *gw, float *gb, long R, int K, int N, hipStream_t s)
 {
-    const int nb = (int)((R + GROUP - 1) / GROUP), nw = (int)((R + WROWS - 1) / WROWS), full = (int)(R / WROWS);
+    const int wrows = weight_rows(R, K, N);
+    const int nb = (int)((R + GROUP - 1) / GROUP), nw = (int)((R + wrows - 1) / wrows), full = (int)(R / wrows);
     if (N % 4 == 0 && vec4(gy, 0, 0, 4) && vec4(pre, 0, 0, 4) && vec4(gz, 0, 0, 4) && vec4(gzb, 0, 0, 2) &&
         vec4(bpart, 0, 0, 4))
         hipLaunchKernelGGL(layer_grad_kernel<4>, dim3(nb), dim3(256), 0, s, gy, pre, gz, (unsigned short *)gzb, bpart,
@@ -652,10 +671,10 @@ void linear_grads(const float *gy, const float *pre, const void *xb, float *gz, 
         g.A = (const unsigned short *)xb + r0 * K;
         g.B = (const unsigned short *)gzb + r0 * N;
         g.C = out;
-        g.sAz = (long)WROWS * K;
+        g.sAz = (long)wrows * K;
         g.sAm = 1;
         g.sAk = K;
-        g.sBz = (long)WROWS * N;
+        g.sBz = (long)wrows * N;
         g.sBk = N;
         g.sBn = 1;
         g.sCz = (long)K * N;
@@ -674,11 +693,16 @@ void linear_grads(const float *gy, const float *pre, const void *xb, float *gz, 
             launch_gemm(h, batch - z < 65535 ? batch - z : 65535, s);
         }
     };
-    if (full) part(0, WROWS, full, wpart);
-    if (nw > full) part((long)full * WROWS, (int)(R - (long)full * WROWS), 1, wpart + (long)full * K * N);
-    const int wblocks = (K * N + 63) / 64;
-    hipLaunchKernelGGL(layer_reduce_kernel, dim3(wblocks + (N + 63) / 64), dim3(1024), 0, s, wpart, nw, K * N, gw,
-                       bpart, nb, N, gb, wblocks);
+    if (full) part(0, wrows, full, wpart);
+    if (nw > full) part((long)full * wrows, (int)(R - (long)full * wrows), 1, wpart + (long)full * K * N);
+    auto reduce = [&](auto kernel, int cols) {
+        const int wblocks = (K * N + cols - 1) / cols;
+        hipLaunchKernelGGL(kernel, dim3(wblocks + (N + cols - 1) / cols), dim3(1024), 0, s, wpart, nw, K * N, gw, bpart,
+                           nb, N, gb, wblocks);
+    };
+    if (nw >= 64) reduce(layer_reduce_kernel<16>, 64);
+    else if (nw > 16) reduce(layer_reduce_kernel<4>, 256);
+    else reduce(layer_reduce_kernel<1>, 1024);
 }
 
 int check_layer(long B, long H, long W, long C, long m)
@@ -923,6 +947,11 @@ extern "C" int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *L, void *stream
     rc = cgfd_fno_gemm_bf16(L->fw, 0, 1, W, L->t3, 2 * mC, C, 1, L->gv, (long)W * C, C, W, C, 2 * m, B * H, 0, stream);
     if (rc) return rc;
     return cgfd_fno_gemm_bf16(L->gzb, 0, C, 1, L->wb, 0, 1, C, L->gv, 0, C, (int)R, C, C, 1, 1, stream);
+}
+
+extern "C" int cgfd_fno_weight_rows(long R, int K, int N)
+{
+    return R <= 0 || K <= 0 || N <= 0 ? CGFD_FNO_EINVAL : weight_rows(R, K, N);
 }
 
 extern "C" int cgfd_fno_linear_bwd(const float *gy, const float *pre, const void *xb, const void *wb, float *gz,

@@ -44,7 +44,7 @@ typedef struct cgfd_fno_fourier_grad {
     void *g;                         /* scratch, bf16 [P, B, 2C] */
     void *t1, *t2, *t3;              /* scratch as in the forward call */
     float *gwr;                      /* scratch [P, 2C, 2C] */
-    float *wpart, *bpart;            /* scratch ceil(R/256)*C*C, ceil(R/128)*C */
+    float *wpart, *bpart;            /* scratch as of cgfd_fno_linear_bwd with K = N = C */
     float *gv, *gwre, *gwim, *gw, *gb;
 } cgfd_fno_fourier_grad;
 int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *layer, void *stream);
@@ -58,10 +58,14 @@ int cgfd_fno_linear_fwd(const void *xb, const void *wb, const float *bias, float
  * bf16: gz = gy * GELU'(pre) (pre null: gy), in bf16 into gzb and on request
  * (the gradient of d) into gz; gx = gz w^T unless null, gw = x^T gz, gb = the
  * column sums of gz in fp32.  N is at most 256.  Scratch:
- * wpart ceil(R/256)*K*N, bpart ceil(R/128)*N fp32 elements. */
+ * wpart ceil(R/rows)*K*N, rows = cgfd_fno_weight_rows(R, K, N), and bpart
+ * ceil(R/128)*N fp32 elements. */
 int cgfd_fno_linear_bwd(const float *gy, const float *pre, const void *xb, const void *wb, float *gz, void *gzb,
                         float *wpart, float *bpart, float *gx, float *gw, float *gb, long R, int K, int N,
                         void *stream);
+
+/* Rows that one partial sum of the weight gradient covers (256 or 512). */
+int cgfd_fno_weight_rows(long R, int K, int N);
 
 /* The network's 13 input fields [n, wi, wj, 13] of n sources at the surface
  * points (i0 + i, j0 + j)*dh: src is n rows of 10 doubles on the device (x, y,

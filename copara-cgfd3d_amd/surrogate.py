@@ -67,9 +67,11 @@ def load_library():
         lib.cgfd_fno_linear_bwd.argtypes = [P] * 11 + [L, I, I, P]
         lib.cgfd_fno_fourier_fwd.argtypes = lib.cgfd_fno_fourier_bwd.argtypes = [P, P]
         lib.cgfd_fno_linear_fwd.argtypes = [P, P, P, P, I, P, L, I, I, P]
+        lib.cgfd_fno_weight_rows.argtypes = [L, I, I]
         lib.cgfd_fno_encode.argtypes = [P, P, I, I, I, I, I, D, D, P]
         for fn in ("cgfd_fno_gemm_bf16", "cgfd_fno_gemm_bf16_ex", "cgfd_fno_gelu_bwd", "cgfd_fno_adam", "cgfd_fno_encode",
-                   "cgfd_fno_linear_fwd", "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd"):
+                   "cgfd_fno_linear_fwd", "cgfd_fno_linear_bwd", "cgfd_fno_fourier_fwd", "cgfd_fno_fourier_bwd",
+                   "cgfd_fno_weight_rows"):
             getattr(lib, fn).restype = I
         _LIB = lib
     return _LIB
@@ -224,7 +226,12 @@ class _Matmul(torch.autograd.Function):
         return gx[:, :ctx.k], _weight_grad(xb, gyb)[:ctx.k]
 
 
-WROWS, GROUP = 256, 128  # rows per partial sum of a layer's weight and bias gradients (cgfd_fno_linear_bwd)
+GROUP = 128  # rows per partial sum of a layer's bias gradient (cgfd_fno_linear_bwd)
+
+
+def _weight_parts(R, K, N):
+    """How many partial sums cgfd_fno_linear_bwd makes of a weight gradient."""
+    return -(-R // load_library().cgfd_fno_weight_rows(R, K, N))
 
 
 def _ptr(t):
@@ -241,7 +248,7 @@ def _linear_grads(gy, pre, xb, wb, want_gx, gz=None):
     (R, K), N, dev = xb.shape, wb.shape[1], gy.device
     new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
     gzb, gx = new(R, N, dtype=torch.bfloat16), new(R, K) if want_gx else None
-    gw, gb, wpart, bpart = new(K, N), new(N), new(-(-R // WROWS) * K * N), new(-(-R // GROUP) * N)
+    gw, gb, wpart, bpart = new(K, N), new(N), new(_weight_parts(R, K, N) * K * N), new(-(-R // GROUP) * N)
     rc = load_library().cgfd_fno_linear_bwd(_ptr(gy), _ptr(pre), _ptr(xb), _ptr(wb), _ptr(gz), _ptr(gzb), _ptr(wpart),
                                             _ptr(bpart), _ptr(gx), _ptr(gw), _ptr(gb), R, K, N, _stream())
     if rc != 0:
@@ -369,7 +376,7 @@ def _fourier_bwd(gy, kept, dims):
     new = lambda *n, dtype=torch.float32: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
     gzb, g = new(R, C, dtype=bf), new(P, B, 2 * C, dtype=bf)
     t1, t2, t3 = new(2 * B * H * m * C, dtype=bf), new(4 * B * m * m * C, dtype=bf), new(2 * B * H * m * C, dtype=bf)
-    gwr, wpart, bpart = new(P, 2 * C, 2 * C), new(-(-R // WROWS) * C * C), new(-(-R // GROUP) * C)
+    gwr, wpart, bpart = new(P, 2 * C, 2 * C), new(_weight_parts(R, C, C) * C * C), new(-(-R // GROUP) * C)
     gv, gwre, gwim, gw, gb = new(R, C), new(P, C, C), new(P, C, C), new(C, C), new(C)
     arg = _Backward(B, H, W, C, m, 0, _ptr(gy), _ptr(pre), _ptr(vb), *(_ptr(t) for t in dft_matrices(H, W, m, dev)),
                     _ptr(wr), _ptr(wb), _ptr(x), _ptr(gzb), _ptr(g), _ptr(t1), _ptr(t2), _ptr(t3), _ptr(gwr),

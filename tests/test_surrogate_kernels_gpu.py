@@ -210,3 +210,21 @@ def test_encode_on_the_device(n, window):
     exact = [c for c in range(13) if c not in (4, 7)]
     assert np.array_equal(got[..., exact], want[..., exact])
     assert (np.abs(got - want) <= EPS * np.abs(want)).all()
+
+
+# one row past 256 and 512 rows, parts summed in 1, 4 and 16 slices and at the
+# edges between them, parts of 512 rows; with GELU, against 64-bit sums of what the
+# GELU backward gives
+@pytest.mark.parametrize("R,K,N,parts", [(257, 8, 4, 2), (1025, 8, 7, 5), (4096, 16, 8, 16), (4097, 16, 8, 17), (16128, 8, 8, 63),
+                                         (16129, 8, 8, 64), (1025, 32768, 256, 3), (24065, 700, 256, 48)])
+def test_weight_gradient_of_any_number_of_parts(R, K, N, parts):
+    assert surrogate._weight_parts(R, K, N) == parts
+    x, w, b, gy = _rand((R, K), 1), _rand((K, N), 2) * K ** -0.5, _rand((N,), 3), _rand((R, N), 4).cuda()
+    t = [v.cuda().requires_grad_() for v in (x, w, b)]
+    y = surrogate.linear(*t, "mfma", gelu=True)
+    pre = y.grad_fn.saved_tensors[2]
+    y.backward(gy)
+    gz, gzb = (v.double().cpu() for v in surrogate.gelu_backward(gy, pre))
+    x = x.bfloat16().double()
+    assert ((t[1].grad.double().cpu() - x.t() @ gzb).abs() <= (R + 4) * EPS * (x.abs().t() @ gzb.abs())).all()
+    assert ((t[2].grad.double().cpu() - gz.sum(0)).abs() <= (R + 4) * EPS * gz.abs().sum(0)).all()
