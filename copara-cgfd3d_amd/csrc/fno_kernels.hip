@@ -275,6 +275,13 @@ bool vec4(const void *p, long sz, long sm, int elem)
     return p == nullptr || ((reinterpret_cast<unsigned long>(p) % (4 * elem)) == 0 && sz % 4 == 0 && sm % 4 == 0);
 }
 
+// what a layer's kernels access 16 bytes at a time without another way (null
+// where a pointer is optional)
+template <typename... P> bool aligned16(P... p)
+{
+    return ((reinterpret_cast<unsigned long>(p) | ...) & 15) == 0;
+}
+
 // staging mode of an operand: unit stride along k (STAGE_K) or along its
 // rows (STAGE_MN), with a 16-byte aligned base and the other strides in
 // multiples of 8 elements; otherwise element by element
@@ -876,6 +883,12 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
     if (!L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wre || !L->wim || !L->w || !L->bias || !L->wr || !L->wb ||
         !L->t1 || !L->x || !L->t2 || !L->t3 || !L->yb)
         return CGFD_FNO_EINVAL;
+    if (!aligned16(L->vb, L->fw, L->gh, L->gi, L->fi, L->wre, L->wim, L->wr, L->wb, L->x, L->t1, L->t2, L->t3, L->y, L->pre,
+                   L->yb))
+        return CGFD_FNO_EINVAL;
+    // the last two products in one launch where whole groups of eight can be staged
+    const bool pair = m % 4 == 0 && vec4(L->bias, 0, 0, 4);
+    if (!pair && (!L->sp || !L->y)) return CGFD_FNO_EINVAL;
     const hipStream_t s = (hipStream_t)stream;
     const long mC = (long)m * C, C2 = 2L * C;
     const long n4 = (long)P * C * C / 4;
@@ -893,15 +906,13 @@ extern "C" int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *L, void *stream)
     // t3 [b][(h,ri)][(kw,c)]
     product_bf16({L->gi, 0, 4L * m, 1}, {L->t2, 4 * m * mC, 1, mC}, rows(L->t3, 2 * H * mC, mC), 2 * H, m * C, 4 * m, B,
                  s);
-    // both in one launch where whole groups of eight can be staged
-    if (m % 4 == 0 && vec4(L->bias, 0, 0, 4)) {
+    if (pair) {
         PairArgs g{(const unsigned short *)L->fi, (const unsigned short *)L->t3, (const unsigned short *)L->vb,
                    (const unsigned short *)L->wb, 2 * m, 1, 2 * mC, C, (long)W * C, C, 1, C, W, C, 2 * m, C,
                    L->gelu ? CGFD_FNO_ACT_GELU : CGFD_FNO_ACT_NONE, L->bias, L->y, L->pre, (unsigned short *)L->yb};
         launch_pair<0>(g, B * H, s);
         return hipGetLastError() == hipSuccess ? 0 : CGFD_FNO_EHIP;
     }
-    if (!L->sp || !L->y) return CGFD_FNO_EINVAL;
     rc = cgfd_fno_gemm_bf16(L->fi, 0, 2 * m, 1, L->t3, 2 * mC, C, 1, L->sp, (long)W * C, C, W, C, 2 * m, B * H, 0,
                             stream);
     if (rc) return rc;
@@ -918,6 +929,9 @@ extern "C" int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *L, void *stream
     if (!L->gy || !L->vb || !L->fw || !L->gh || !L->gi || !L->fi || !L->wr || !L->wb || !L->x || !L->gzb || !L->t1 ||
         !L->g || !L->t2 || !L->t3 || !L->gwr || !L->wpart || !L->bpart || !L->gv || !L->gwre || !L->gwim || !L->gw ||
         !L->gb)
+        return CGFD_FNO_EINVAL;
+    if (!aligned16(L->vb, L->fw, L->gh, L->gi, L->fi, L->wr, L->wb, L->x, L->gzb, L->g, L->t1, L->t2, L->t3, L->gwr, L->gv,
+                   L->gwre, L->gwim))
         return CGFD_FNO_EINVAL;
     const hipStream_t s = (hipStream_t)stream;
     const long mC = (long)m * C, C2 = 2L * C, R = (long)B * H * W;

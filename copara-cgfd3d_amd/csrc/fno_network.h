@@ -18,7 +18,8 @@ extern "C" {
  * in bf16 only (the operand of the next product) and stored in the order that
  * the next product reads.  C is a multiple of 8 and at most 256, B*H at most
  * 65535.  fw, gh, gi, fi: the bf16 DFT matrices [2m, W], [4m, 2H], [2H, 4m],
- * [W, 2m].  Sizes in elements, R = B*H*W, P = 2*modes*modes. */
+ * [W, 2m].  Sizes in elements, R = B*H*W, P = 2*modes*modes.  Every pointer but w,
+ * bias and sp is aligned to 16 bytes. */
 typedef struct cgfd_fno_fourier {
     int B, H, W, C, modes, gelu;
     const void *vb;                  /* v in bf16 [R, C] */
@@ -35,7 +36,8 @@ typedef struct cgfd_fno_fourier {
 int cgfd_fno_fourier_fwd(const cgfd_fno_fourier *layer, void *stream);
 
 /* Its backward: gv, gwre, gwim, gw, gb from gy.  vb, wr, wb, x and pre as the
- * forward call had or wrote them (pre null without GELU). */
+ * forward call had or wrote them (pre null without GELU).  Every pointer but gy,
+ * pre, wpart, bpart, gw and gb is aligned to 16 bytes. */
 typedef struct cgfd_fno_fourier_grad {
     int B, H, W, C, modes, unused;
     const float *gy, *pre;
@@ -50,7 +52,8 @@ typedef struct cgfd_fno_fourier_grad {
 int cgfd_fno_fourier_bwd(const cgfd_fno_fourier_grad *layer, void *stream);
 
 /* yb = act(x w + bias) in bf16 only, x [R, K] and w [K, N] in bf16, N a multiple
- * of 4; the value before the activation into pre unless null. */
+ * of 4; the value before the activation into pre unless null.  bias and pre are
+ * aligned to 16 bytes, yb to 8. */
 int cgfd_fno_linear_fwd(const void *xb, const void *wb, const float *bias, float *pre, int act, void *yb, long R,
                         int K, int N, void *stream);
 

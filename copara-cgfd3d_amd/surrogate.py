@@ -238,6 +238,13 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def _aligned(t):
+    """t contiguous at an address that 16-byte accesses can use: a copy of what
+    is not, such as a view into a flat buffer of parameters."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def _stream():
     return torch.cuda.current_stream().cuda_stream
 
@@ -262,8 +269,7 @@ def _linear_bf16(xb, wb, b, gelu, keep):
     R, (K, N) = xb.shape[0], wb.shape
     yb = torch.empty(R, N, device=xb.device, dtype=torch.bfloat16)
     pre = torch.empty(R, N, device=xb.device) if gelu and keep else None
-    b = b.contiguous()
-    b = b.clone() if b.data_ptr() % 16 else b
+    b = _aligned(b)
     rc = load_library().cgfd_fno_linear_fwd(_ptr(xb), _ptr(wb), _ptr(b), _ptr(pre), ACT_GELU if gelu else ACT_NONE,
                                             _ptr(yb), R, K, N, _stream())
     if rc != 0:
@@ -351,8 +357,7 @@ def _fourier_fwd(vb, wre, wim, w, b, dims, gelu, keep, want_y):
     without it."""
     B, H, W, C, m = dims
     R, P, dev = B * H * W, 2 * m * m, vb.device
-    wre, wim, w, b = (t.contiguous() for t in (wre, wim, w, b))
-    b = b.clone() if b.data_ptr() % 16 else b
+    wre, wim, w, b = (_aligned(t) for t in (wre, wim, w, b))
     new = lambda *n, dtype=torch.bfloat16: torch.empty(*n, device=dev, dtype=dtype)  # noqa: E731
     wr, wb, x = new(P, 2 * C, 2 * C), new(C, C), new(P, B, 2 * C)
     t1, t2, t3 = new(2 * B * H * m * C), new(4 * B * m * m * C), new(2 * B * H * m * C)
@@ -393,11 +398,6 @@ def _native(x, *params):
     not takes the general path, which converts or refuses it."""
     return x.is_cuda and all(p.dtype == torch.float32 and p.device == x.device and tuple(p.shape) == shape
                              for p, shape in params)
-
-
-def _aligned(gy):
-    gy = gy.contiguous()
-    return gy.clone() if gy.data_ptr() % 16 else gy
 
 
 class _Trunk(torch.autograd.Function):

@@ -228,3 +228,27 @@ def test_weight_gradient_of_any_number_of_parts(R, K, N, parts):
     x = x.bfloat16().double()
     assert ((t[1].grad.double().cpu() - x.t() @ gzb).abs() <= (R + 4) * EPS * (x.abs().t() @ gzb.abs())).all()
     assert ((t[2].grad.double().cpu() - gz.sum(0)).abs() <= (R + 4) * EPS * gz.abs().sum(0)).all()
+
+
+# parameters that are views into one flat buffer, at every offset within 16 bytes
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("modes", [4, 3])
+def test_parameters_in_a_flat_buffer(off, modes):
+    net = surrogate.FNO2d(surrogate.NCH, 3, 16, modes, 2, proj=32, seed=3).cuda()
+    x, gy = _rand((2, 12, 16, surrogate.NCH), 1).cuda(), _rand((2, 12, 16, 3), 2).cuda()
+    y = net(x)
+    y.backward(gy)
+    want = {n: p.grad.clone() for n, p in net.named_parameters()}
+    flat = torch.zeros(off + sum(p.numel() + 4 for p in net.parameters()), device="cuda")
+    at = off
+    for p in net.parameters():
+        view = flat[at:at + p.numel()].view(p.shape)
+        view.copy_(p.detach())
+        p.data, p.grad = view, None
+        at += -(-p.numel() // 4) * 4
+    assert all(p.data_ptr() % 16 == 4 * off for p in net.parameters())
+    y2 = net(x)
+    y2.backward(gy)
+    assert torch.equal(y2, y)
+    for n, p in net.named_parameters():
+        assert torch.equal(p.grad, want[n]), n
