@@ -1032,17 +1032,20 @@ def encode(base, src):
 
 def encode_device(base, src, device):
     """encode's fields as a tensor on `device`, computed there when it is a GPU
-    (the same operations in double, rounded once to fp32)."""
-    if torch.device(device).type != "cuda" or not 0 < len(src) <= 65535:
-        return torch.from_numpy(encode(base, src)).to(device)
+    (the same operations in double, rounded once to fp32).  As there, columns
+    past the tenth are not read; what the kernel does not take (no source, more
+    than 65535, rows without log10 M0, an empty window) is encoded on the host."""
     i0, j0, wi, wj = _window(base)
-    rows = torch.from_numpy(np.ascontiguousarray(src, dtype=np.float64)).to(device)
-    if rows.shape[1] != 10:
-        raise SurrogateError("source rows have 10 columns (see source_rows)")
-    out = torch.empty(len(src), wi, wj, NCH, device=device, dtype=torch.float32)
+    L = max(base["ni"], base["nj"]) * base["dh"]
+    rows = np.asarray(src, np.float64)
+    if (torch.device(device).type != "cuda" or rows.ndim != 2 or rows.shape[1] < 10 or not 0 < len(rows) <= 65535
+            or wi * wj == 0 or not L > 0):
+        return torch.from_numpy(encode(base, src)).to(device)
+    rows = torch.from_numpy(np.array(rows[:, :10], order="C")).to(device)  # a copy: the caller's may be read-only
+    out = torch.empty(len(rows), wi, wj, NCH, device=device, dtype=torch.float32)
     with torch.cuda.device(out.device):
-        rc = load_library().cgfd_fno_encode(_ptr(rows), _ptr(out), len(src), i0, j0, wi, wj, float(base["dh"]),
-                                            max(base["ni"], base["nj"]) * base["dh"], _stream())
+        rc = load_library().cgfd_fno_encode(_ptr(rows), _ptr(out), len(rows), i0, j0, wi, wj, float(base["dh"]), float(L),
+                                            _stream())
     if rc != 0:
         raise SurrogateError(f"cgfd_fno_encode returned {rc}")
     return out

@@ -252,3 +252,32 @@ def test_parameters_in_a_flat_buffer(off, modes):
     assert torch.equal(y2, y)
     for n, p in net.named_parameters():
         assert torch.equal(p.grad, want[n]), n
+
+
+# rows that the host encodes as well: further columns, a column order of their
+# own, a read-only array, a list of rows, no log10 M0, an empty window
+@pytest.mark.filterwarnings("error")
+@pytest.mark.parametrize("form", ["wide", "fortran", "read-only", "list", "nine", "empty window"])
+def test_encode_on_the_device_takes_what_the_host_takes(form):
+    base = dict(ni=20, nj=20, dh=100, window=(3, 3, 0 if form == "empty window" else 14))
+    rng = np.random.default_rng(2)
+    rows = np.concatenate([rng.uniform(0, 2000, (3, 2)), rng.uniform(500, 3000, (3, 1)), rng.uniform(-1, 1, (3, 9))], 1)
+    src = dict(wide=rows, fortran=np.asfortranarray(rows[:, :10]), list=[r for r in rows[:, :10]], nine=rows[:, :9]).get(form, rows[:, :10].copy())
+    if form == "read-only":
+        src.flags.writeable = False
+    want, got = surrogate.encode(base, src), surrogate.encode_device(base, src, "cuda").cpu().numpy()
+    assert got.shape == want.shape
+    assert (np.abs(got - want) <= EPS * np.abs(want)).all()
+
+
+def test_predict_takes_rows_with_further_columns():
+    base = dict(ni=24, nj=24, nk=20, dh=100.0, dt=0.006, nt=8, nabs=[3] * 5 + [0], window=(0, 0, 24),
+                stations=np.zeros((0, 2), np.int64), depth_cells=(10, 36))
+    sur = surrogate.Surrogate(base, 16, 4, 2)
+    sur.mu, sur.sd = -16.0, 0.8
+    rng = np.random.default_rng(3)
+    rows = surrogate.source_rows(rng.uniform([500, 500, 900, 0, 10, -180, 14], [1900, 1900, 1700, 360, 90, 180, 17], (3, 7)))
+    want = sur.predict(rows, rows=True)
+    got = sur.predict(np.concatenate([rows, np.ones((3, 2))], 1), rows=True)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
