@@ -87,14 +87,13 @@ def _span_ok(t, offsets):
 ACT_NONE, ACT_GELU = 0, 1
 
 
-def _pad_cols(t, n):
-    """n zero columns on the right (none: t itself, without the copy that
-    torch's pad would make)."""
-    return torch.nn.functional.pad(t, (0, n)) if n else t
-
-
-def _pad_rows(t, n):
-    return torch.nn.functional.pad(t, (0, 0, 0, n)) if n else t
+def _operand(t, rows=0, cols=0):
+    """t in bf16 with this many zero rows below and columns on the right: a
+    tensor of its own also where t is bf16 already, since a backward reads it
+    after the caller may have changed t, and one copy in any case but a padded
+    one."""
+    tb = t.to(torch.bfloat16, copy=not (rows or cols))
+    return torch.nn.functional.pad(tb, (0, cols, 0, rows)) if rows or cols else tb
 
 
 def _as3(t):
@@ -209,8 +208,8 @@ class _Matmul(torch.autograd.Function):
     def forward(ctx, x, w):
         K = x.shape[1]
         pad = -K % 8
-        xb = _pad_cols(x.to(torch.bfloat16), pad).contiguous()
-        wb = _pad_rows(w.to(torch.bfloat16), pad).contiguous()
+        xb = _operand(x, cols=pad).contiguous()
+        wb = _operand(w, rows=pad).contiguous()
         y = torch.empty(x.shape[0], w.shape[1], device=x.device, dtype=torch.float32)
         gemm(xb, wb, y)
         ctx.save_for_backward(xb, wb)
@@ -290,9 +289,9 @@ class _Linear(torch.autograd.Function):
         K = x.shape[1]
         pad = -K % 8
         if xb is None or pad:  # a producer's bf16 copy serves as the operand when no padding is needed
-            xb = _pad_cols(x.to(torch.bfloat16), pad)
+            xb = _operand(x, cols=pad)
         xb = xb.contiguous()
-        wb = _pad_rows(w.to(torch.bfloat16), pad).contiguous()
+        wb = _operand(w, rows=pad).contiguous()
         y = torch.empty(x.shape[0], w.shape[1], device=x.device, dtype=torch.float32)
         pre = torch.empty_like(y) if gelu and keep else None
         yb = torch.empty(y.shape, device=x.device, dtype=torch.bfloat16) if want_bf16 else None
@@ -415,8 +414,8 @@ class _Trunk(torch.autograd.Function):
     def forward(ctx, x, dims, keep, *params):
         K = x.shape[1]
         pad = -K % 8
-        xb = _pad_cols(x.to(torch.bfloat16), pad).contiguous()
-        lw = _pad_rows(params[0].to(torch.bfloat16), pad).contiguous()
+        xb = _operand(x, cols=pad).contiguous()
+        lw = _operand(params[0], rows=pad).contiguous()
         vb, _ = _linear_bf16(xb, lw, params[1], False, keep)
         layers, y, saved = (len(params) - 2) // 4, None, [xb, lw]
         for l in range(layers):
@@ -451,7 +450,7 @@ class _Head(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, v, vb, w1, b1, w2, b2, keep):
-        vb = (v.to(torch.bfloat16) if vb is None else vb).contiguous()
+        vb = (_operand(v) if vb is None else vb).contiguous()
         w1b, w2b = w1.to(torch.bfloat16).contiguous(), w2.to(torch.bfloat16).contiguous()
         hb, pre = _linear_bf16(vb, w1b, b1, True, keep)
         y = torch.empty(v.shape[0], w2.shape[1], device=v.device, dtype=torch.float32)
