@@ -233,12 +233,15 @@ static long plane_tiles(const cgfd_ctx *c, int tw)
 // 295 us at 64 (192 lanes), 244 at 32 (160).  A grid too small to fill the chip
 // gains nothing from fewer lanes and keeps 64 there.
 static bool narrow_pays(long lanes64, long lanes32) { return lanes64 * 100 > lanes32 * 108; }
+static int auto_tile_width(const cgfd_ctx *c)
+{
+    if (c->prec == CGFD_FP64 && 2 * plane_tiles(c, 64) * c->g.nk <= kFewBlocks) return 64;
+    return narrow_pays((c->g.ni + 63) / 64 * 64, (c->g.ni + 31) / 32 * 32) ? 32 : 64;
+}
 static int tile_width(const cgfd_ctx *c)
 {
     if (c->tile_w) return c->tile_w;
-    if (c->tile_pref) return c->tile_pref;
-    if (c->prec == CGFD_FP64 && 2 * plane_tiles(c, 64) * c->g.nk <= kFewBlocks) return 64;
-    return narrow_pays((c->g.ni + 63) / 64 * 64, (c->g.ni + 31) / 32 * 32) ? 32 : 64;
+    return c->tile_pref ? c->tile_pref : auto_tile_width(c);
 }
 
 // z chunks per column sweep: about 2048 tiles in the launch (4096 workgroups,
@@ -1962,7 +1965,8 @@ int cgfd_set_tile_width(cgfd_ctx *c, int width)
 {
     if (!c) return CGFD_EINVAL;
     if (width != 0 && width != 32 && width != 64) return fail(c, CGFD_EINVAL, "tile width must be 0, 32 or 64");
-    if (width == 32 && c->prec == CGFD_FP64) return fail(c, CGFD_EINVAL, "the FP64 kernels run 64-column tiles");
+    if (width == 32 && c->prec == CGFD_FP64 && auto_tile_width(c) != 32)
+        return fail(c, CGFD_EINVAL, "FP64 takes 64-column tiles on this grid (32 only where that is the automatic width)");
     if (width != c->tile_w) {
         c->tile_w = width;
         c->args_dirty = true; // the next run rewrites the image and drops captured cycles

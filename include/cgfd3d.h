@@ -264,12 +264,13 @@ int cgfd_profile_read(cgfd_ctx *ctx, double *ms_stage, long *n_stage, double *ms
 /* Launch shape of the fused stage kernel: z-chunks per column sweep and
  * rows per workgroup (0 keeps the current value). */
 int cgfd_set_tuning(cgfd_ctx *ctx, int zchunks, int rows);
-/* Tile width of the default (LDS) stage kernel, no reference counterpart:
+/* Tile width of the default stage kernel, no reference counterpart:
  * 64 columns x 4 rows per workgroup, or 32 x 8, which leaves fewer lanes idle
  * on rows whose length is 1-32 past a multiple of 64 (80 cells: 96 lanes
- * instead of 128) but costs about 6 % more per lane.  0 (the default) takes
+ * instead of 128) but costs 2-4 % more per lane.  0 (the default) takes
  * 32 when 64-column tiles need over 8 % more lanes (in FP64 on grids that
- * fill the chip); FP64 contexts take 0 or 64.  Results do not depend on it.
+ * fill the chip); FP64 contexts take 32 only where the default does.
+ * Results do not depend on it.
  * cgfd_tile_width returns the width the next launch uses. */
 int cgfd_set_tile_width(cgfd_ctx *ctx, int width);
 int cgfd_tile_width(const cgfd_ctx *ctx);

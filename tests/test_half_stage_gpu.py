@@ -97,3 +97,18 @@ def test_chunks_of_a_launch_just_past_one_round(ni, nj, nk, shear, chunks):
     assert g.autotune() == chunks  # with one step there is nothing to time: the default choice
     g.close()
     _compare(sc, 1, 32)
+
+
+# the width that a context reports can be set on it, in either precision
+@pytest.mark.parametrize("prec", [cgfd3d.FP32, cgfd3d.FP64])
+@pytest.mark.parametrize("ni,nj,nk,width", [(80, 40, 20, 32), (200, 64, 40, 32), (64, 40, 20, 64), (128, 64, 40, 64)])
+def test_reported_tile_width_can_be_set(prec, ni, nj, nk, width):
+    g = cgfd3d.Simulation(ni, nj, nk, 100.0, 0.005, 4, precision=prec)
+    assert g.tile_width() == width
+    for w in (width, 64, 0, width):
+        g.set_tile_width(w)
+        assert g.tile_width() == (w or width)
+    if prec == cgfd3d.FP64 and width == 64:
+        with pytest.raises(cgfd3d.CgfdError, match="64-column"):
+            g.set_tile_width(32)
+    g.close()
