@@ -1284,7 +1284,7 @@ static bool batch_fusable(cgfd_ctx *const *ctxs, int n)
     if (n < 2 || n > 4096) return false; // 9 traction-image parts per grid in a 65535 grid.z
     const cgfd_ctx *c0 = ctxs[0];
     auto hm = [](const cgfd_ctx *c) { return c->hmet && c->use_hmet; };
-    long most = 0; // workgroups at the most z chunks batch_layout can pick
+    long most = 0; // tiles at the most z chunks batch_layout can pick
     for (int i = 0; i < n; i++) {
         const cgfd_ctx *c = ctxs[i];
         if (c->prof || c->variant != 0) return false;
@@ -1295,23 +1295,25 @@ static bool batch_fusable(cgfd_ctx *const *ctxs, int n)
         for (int j = 0; j < i; j++)
             if (ctxs[j] == c) return false; // a grid listed twice would be stepped twice per launch
     }
-    return most < 0x7fffffffL;
+    // a launch counts its lanes along x in 32 bits: two workgroups of 64 per tile
+    return most <= (0xffffffffL / 64) / 2;
 }
 
-// Workgroups of a batched stage launch (the grids of one tile width tw):
-// every grid sweeps its columns in about the same number of z chunks, chosen
-// for about CGFD_BATCH_WORKGROUPS workgroups over the launch, with at most
-// ~9 (kChunkPlanes) and at least 2 planes per chunk per grid; a grid whose z-chunk count
-// was tuned (cgfd_autotune, cgfd_set_tuning) keeps its own.  zlen[c] is grid
-// c's chunk length, starts[c] its first workgroup.
-#ifndef CGFD_BATCH_WORKGROUPS
-#define CGFD_BATCH_WORKGROUPS 2048
-#endif
+// Tiles of a batched stage launch (the grids of one tile width tw): every grid
+// sweeps its columns in about the same number of z chunks, chosen for about
+// kBatchTiles tiles (two workgroups each) over the launch, with at most ~9
+// (kChunkPlanes) and at least 2 planes per chunk per grid; a grid whose z-chunk
+// count was tuned (cgfd_autotune, cgfd_set_tuning) keeps its own.  zlen[c] is grid
+// c's chunk length, starts[c] its first tile.  Measured at 9 / 12 / 25 planes, stage
+// and traction image: 32 grids of 80x80x48 711 / 709 / 748 us, 12 of 150x150x100
+// 1487 / 1477 / 1527, 8 of mixed sizes 974 / 984 / 1044, 8 of 192x192x128 1753 / 1753 /
+// 1764; only 32 of 192x192x128 are faster at longer chunks (7.32 / 7.19 / 7.07 ms).
+constexpr int kBatchTiles = 2048;
 static void batch_layout(cgfd_ctx *const *ctxs, int n, int tw, int *zlen, int *starts)
 {
     long tiles = 0;
     for (int i = 0; i < n; i++) tiles += plane_tiles(ctxs[i], tw);
-    const long zc = std::max(1L, (CGFD_BATCH_WORKGROUPS + tiles - 1) / tiles);
+    const long zc = std::max(1L, (kBatchTiles + tiles - 1) / tiles);
     starts[0] = 0;
     for (int i = 0; i < n; i++) {
         const int nk = ctxs[i]->g.nk;
@@ -1325,7 +1327,7 @@ static void batch_layout(cgfd_ctx *const *ctxs, int n, int tw, int *zlen, int *s
 
 // The device side of the allocation-free batch entry point: one fixed
 // array per device for the argument images of up to kStaticBatchMax grids
-// and their workgroup starts.  Host code reaches it only through the
+// and their first tiles.  Host code reaches it only through the
 // address hipGetSymbolAddress returns for the current device.
 constexpr int kStaticBatchMax = 64;
 constexpr size_t kStaticBatchBytes =
@@ -1368,7 +1370,7 @@ template <typename R> static int run_batch_fused(cgfd_ctx *const *ctxs_in, int n
     HIPCHK(c0, hipSetDevice(c0->dev));
     // Every grid runs at its own tile width: the grids of width 64 first,
     // then those of width 32 (group 1), one stage launch per group.  The
-    // workgroup starts of each group begin at 0: group g's table lies at
+    // first tiles of each group begin at 0: group g's table lies at
     // starts + gfirst[g] + g.
     cgfd_ctx *ord_fixed[kStaticBatchMax];
     int zlen[kStaticBatchMax], starts_fixed[kStaticBatchMax + 2];
@@ -1434,7 +1436,7 @@ template <typename R> static int run_batch_fused(cgfd_ctx *const *ctxs_in, int n
         HIPCHK(c0, hipMemcpy(fixed->ptr + sofs, starts, sbytes, hipMemcpyHostToDevice));
         img_d = fixed->ptr;
     } else {
-        // device image: the grids' argument images, then the workgroup starts
+        // device image: the grids' argument images, then their first tiles
         std::vector<char> img(sofs + sbytes);
         for (int i = 0; i < n; i++) make_image<R>(ctxs[i], img.data() + (size_t)i * kCtxArgBytes, zl[i]);
         memcpy(img.data() + sofs, starts, sbytes);
