@@ -254,9 +254,10 @@ static int tile_width(const cgfd_ctx *c)
 // (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
 // 31.2 us at 1 plane, 29.3 at 2).
 // The FP32 kernel that loads all nine metrics holds 3 workgroups per CU (4 with
-// constant horizontal metrics): a launch of 2-plane chunks just past that takes
+// constant horizontal metrics or, in 64-column tiles, a Cartesian part): a launch of 2-plane chunks just past that takes
 // 3 planes if those fit at once (64x64x64 35.4 -> 32.3 us with the traction image,
-// 64x64x50 31.0 -> 29.8, 48x64x70 37.2 -> 32.4, 60x60x60 33.2 both ways).
+// 64x64x50 31.0 -> 29.8, 48x64x70 37.2 -> 32.4, 60x60x60 33.2 both ways; with a
+// Cartesian part 64x64x64 29.6 at 2 planes, 32.3 at 3).
 constexpr int kChunkPlanes = 9;
 constexpr int kNineMetricBlocks = 3 * 256;
 static int default_zchunks(const cgfd_ctx *c)
@@ -267,7 +268,7 @@ static int default_zchunks(const cgfd_ctx *c)
     long zc = std::max((2048 + tiles - 1) / tiles, (long)(nk + kChunkPlanes - 1) / kChunkPlanes);
     const int least = blocks(nk) <= kFewBlocks ? 1 : 2; // planes of the shortest chunk
     zc = std::max(1L, std::min(zc, (long)std::max(1, nk / least)));
-    const bool nine = c->prec == CGFD_FP32 && !(c->hmet && c->use_hmet);
+    const bool nine = c->prec == CGFD_FP32 && !(c->hmet && c->use_hmet) && c->zcon <= 0;
     if (nine && zc == nk / 2 && blocks(zc) > kNineMetricBlocks && blocks((nk + 2) / 3) <= kNineMetricBlocks)
         zc = (nk + 2) / 3;
     return (int)zc;

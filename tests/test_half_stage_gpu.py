@@ -112,3 +112,13 @@ def test_reported_tile_width_can_be_set(prec, ni, nj, nk, width):
         with pytest.raises(cgfd3d.CgfdError, match="64-column"):
             g.set_tile_width(32)
     g.close()
+
+
+# the kernel with a Cartesian part holds as many workgroups as the one for three
+# metrics: 2-plane chunks of the same grid fit at once
+def test_chunks_of_a_hybrid_grid():
+    sc = dict(scenario.config_random(64, 64, 64, 1, [5, 4, 4, 5, 5, 0], seed=9, shear=True), conindex=30)
+    g = cgfd3d.Simulation(64, 64, 64, sc["dh"], sc["dt"], 1)
+    g.setup(sc)
+    assert g.autotune() == 32
+    g.close()
