@@ -86,22 +86,6 @@ template <typename R> __device__ __forceinline__ void stg_once(R *base, unsigned
     stg(base, off, v);
 #endif
 }
-template <typename R> __device__ __forceinline__ R ld_once(const R *p)
-{
-#if CGFD_NT
-    return __builtin_nontemporal_load(p);
-#else
-    return *p;
-#endif
-}
-template <typename R> __device__ __forceinline__ void st_once(R *p, R v)
-{
-#if CGFD_NT
-    __builtin_nontemporal_store(v, p);
-#else
-    *p = v;
-#endif
-}
 
 // member-wise copy of the geometry out of a constant-address-space block
 template <typename AP> __device__ __forceinline__ Geom geom_of(AP a)
@@ -170,33 +154,14 @@ template <typename R> struct CellIn {
     R fw[NF], tw[NF];
 };
 
-// HM = 1: the horizontal metrics are known to be xi_x = eta_y = 1 and
-// xi_y = xi_z = eta_x = eta_z = 0 in every valid cell (grids with fixed x and
-// y spacing, vertically stretched: the reference's vmap meshes,
-// gridmesh.cpp:101-129, 386-393).  Only the three zeta metrics are loaded;
-// the others enter every product as exact constants, so each operation
-// rounds exactly as with the loaded values.  A loaded -0 becomes +0, which
-// can flip the sign of an exactly-zero intermediate but no value: nothing on
-// this path divides by, or otherwise distinguishes, a signed zero.
-template <typename R, int ST, int HM = 0, typename AP>
+template <typename R, int ST, typename AP>
 __device__ __forceinline__ void load_cell(AP a, unsigned pb, long fs, CellIn<R> &in)
 {
     in.lam2mu = ldg_once(a->med, pb);
     in.miu = ldg_once(a->med + fs, pb);
     in.rhoinv = ldg_once(a->med + 2 * fs, pb);
-    if (HM) {
-        in.m[XIX] = (R)1;
-        in.m[XIY] = (R)0;
-        in.m[XIZ] = (R)0;
-        in.m[ETX] = (R)0;
-        in.m[ETY] = (R)1;
-        in.m[ETZ] = (R)0;
 #pragma unroll
-        for (int m = ZTX; m <= ZTZ; ++m) in.m[m] = ldg_once(a->met + m * fs, pb);
-    } else {
-#pragma unroll
-        for (int m = 0; m < 9; ++m) in.m[m] = ldg_once(a->met + m * fs, pb);
-    }
+    for (int m = 0; m < 9; ++m) in.m[m] = ldg_once(a->met + m * fs, pb);
 #pragma unroll
     for (int c = 0; c < NF; ++c) {
         if (ST == 1 || ST == 2) in.fw[c] = ldg_once(a->fw + c * fs, pb);
@@ -254,7 +219,7 @@ __device__ __forceinline__ void store_aux(AP a, int ax, long aidx, const AuxIn<R
 // rates with their RK update, the traction-image override and the point
 // sources.  The RK update of the wavefield is rk_store (below).
 //   w: z window of the stage input (slot CI is the cell itself)
-template <typename R, int SX, int SZ, int ST, int HY, typename AP>
+template <typename R, int SX, int SZ, int ST, typename AP>
 __device__ __forceinline__ void cell_rates(AP a, const Column<R> &k, const CellIn<R> &in, R (&Dx)[NF], R (&Dy)[NF],
                                            R (&Dz)[NF], const R (&w)[NF][5], int x, int y, int z, int &e,
                                            int tindex, R (&hv)[NF])
@@ -303,12 +268,11 @@ __device__ __forceinline__ void cell_rates(AP a, const Column<R> &k, const CellI
     // planes below the conversion depth (z < zcon, uniform over the
     // workgroup) take CalWave's Cartesian form, which uses only xi_x, eta_y
     // and zeta_z in its own operand order (calculate.cu:3910-3956);
-    // elsewhere the curvilinear contraction of CalWaveCL (4855-4930).  HY = 0
-    // compiles the curvilinear form alone (grids without a Cartesian part).
+    // elsewhere the curvilinear contraction of CalWaveCL (4855-4930).
     R DxiVx, DetVx, DztVx, DxiVy, DetVy, DztVy, DxiVz, DetVz, DztVz;
     R DxiTxx, DetTxx, DztTxx, DxiTyy, DetTyy, DztTyy, DxiTzz, DetTzz, DztTzz;
     R DxiTxy, DetTxy, DztTxy, DxiTxz, DetTxz, DztTxz, DxiTyz, DetTyz, DztTyz;
-    if (!HY || z >= a->zcon) {
+    if (z >= a->zcon) {
         DxiVx = (xix * Dx[TXX] + xiy * Dx[TXY] + xiz * Dx[TXZ]) * rho;
         DetVx = (etx * Dy[TXX] + ety * Dy[TXY] + etz * Dy[TXZ]) * rho;
         DztVx = (ztx * Dz[TXX] + zty * Dz[TXY] + ztz * Dz[TXZ]) * rho;
@@ -532,7 +496,8 @@ __device__ __forceinline__ void cell_rates(AP a, const Column<R> &k, const CellI
 // store of the RK update: in FP32 a buffer store whose lane offset lies
 // past the field (keep = false) is dropped by the hardware, so lanes outside
 // the grid store nothing and no branch is needed; FP64 lanes outside the
-// grid store the zeros they computed into their own guard cell
+// grid store the zeros they computed into the guard cell that they read, which
+// several of them share
 template <typename R>
 __device__ __forceinline__ void stg_keep(R *base, unsigned off, R v, bool keep, unsigned bytes)
 {
@@ -550,21 +515,20 @@ __device__ __forceinline__ void stg_keep(R *base, unsigned off, R v, bool keep, 
 // cell's rates hv.  The stage-0 input is FW itself (w[c][CI]).
 template <typename R, int SZ, int ST, typename AP>
 __device__ __forceinline__ void rk_store(AP a, const CellIn<R> &in, const R (&w)[NF][5], const R (&hv)[NF],
-                                         unsigned pb, long fs, bool keep = true)
+                                         unsigned pb, long fs)
 {
     constexpr int CI = SZ > 0 ? 1 : 3;
-    const unsigned fb = (unsigned)(fs * (long)sizeof(R)); // bytes of one field (< 4 GiB)
 #pragma unroll
     for (int c = 0; c < NF; ++c) {
         if (ST == 0) {
             const R f0 = w[c][CI];
-            stg_keep(a->wout + c * fs, pb, f0 + a->alpha * hv[c], keep, fb);
-            stg_keep(a->tw + c * fs, pb, f0 + a->beta * hv[c], keep, fb);
+            stg_once(a->wout + c * fs, pb, f0 + a->alpha * hv[c]);
+            stg_once(a->tw + c * fs, pb, f0 + a->beta * hv[c]);
         } else if (ST < 3) {
-            stg_keep(a->wout + c * fs, pb, in.fw[c] + a->alpha * hv[c], keep, fb);
-            stg_keep(a->tw + c * fs, pb, in.tw[c] + a->beta * hv[c], keep, fb);
+            stg_once(a->wout + c * fs, pb, in.fw[c] + a->alpha * hv[c]);
+            stg_once(a->tw + c * fs, pb, in.tw[c] + a->beta * hv[c]);
         } else {
-            stg_keep(a->wout + c * fs, pb, in.tw[c] + a->beta * hv[c], keep, fb);
+            stg_once(a->wout + c * fs, pb, in.tw[c] + a->beta * hv[c]);
         }
     }
 }
@@ -591,7 +555,7 @@ __device__ __forceinline__ void finish_cell(AP a, const Column<R> &k, const Cell
                                             int &e, long fs, int tindex)
 {
     R hv[NF];
-    cell_rates<R, SX, SZ, ST, 1>(a, k, in, Dx, Dy, Dz, w, x, y, z, e, tindex, hv);
+    cell_rates<R, SX, SZ, ST>(a, k, in, Dx, Dy, Dz, w, x, y, z, e, tindex, hv);
     rk_store<R, SZ, ST>(a, in, w, hv, pb, fs);
     pgv_update<R, ST>(a, k, in, hv, z - (geom_of(a).nk - 3));
 }
@@ -713,6 +677,14 @@ template <typename R, int PART> struct HalfIn {
     R fw[Half<PART>::NO], tw[Half<PART>::NO];
 };
 
+// HM = 1: the horizontal metrics are known to be xi_x = eta_y = 1 and
+// xi_y = xi_z = eta_x = eta_z = 0 in every valid cell (grids with fixed x and
+// y spacing, vertically stretched: the reference's vmap meshes,
+// gridmesh.cpp:101-129, 386-393).  Only the three zeta metrics are loaded;
+// the others enter every product as exact constants, so each operation
+// rounds exactly as with the loaded values.  A loaded -0 becomes +0, which
+// can flip the sign of an exactly-zero intermediate but no value: nothing on
+// this path divides by, or otherwise distinguishes, a signed zero.
 template <typename R, int ST, int HM, int PART, typename AP>
 __device__ __forceinline__ void load_half(AP a, unsigned pb, long fs, HalfIn<R, PART> &in)
 {
