@@ -508,9 +508,9 @@ def main():
     ap.add_argument("--rows", type=int, default=0)
     ap.add_argument("--graph", action="store_true", help="replay captured 4-step cycles (cgfd_set_graph)")
     ap.add_argument("--variant", type=int, default=0,
-                    help="stage kernel: 0 = LDS-staged planes, 1 = direct loads, 2 = split velocity/stress")
+                    help="stage kernel: 0 = default (half the system per workgroup), 1 = direct loads, 2 = split velocity/stress")
     ap.add_argument("--tile-width", type=int, default=0, choices=[0, 32, 64],
-                    help="tile width of the LDS stage kernel (0: the one the grid's rows pick)")
+                    help="tile width of the default stage kernel (0: the one the grid's rows pick)")
     ap.add_argument("--copy-mib", type=int, default=0,
                     help="after the timed steps, run a plain device copy of this many MiB (counter calibration)")
     args = ap.parse_args()

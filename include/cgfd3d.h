@@ -274,9 +274,10 @@ int cgfd_set_tuning(cgfd_ctx *ctx, int zchunks, int rows);
  * cgfd_tile_width returns the width the next launch uses. */
 int cgfd_set_tile_width(cgfd_ctx *ctx, int width);
 int cgfd_tile_width(const cgfd_ctx *ctx);
-/* Stage kernel variant: 0 = xy planes staged in LDS (default), 1 = in-plane
- * stencil taps loaded directly through the vector caches.  Both produce
- * identical results. */
+/* Stage kernel variant: 0 = two workgroups per tile, one for the velocities and
+ * one for the stresses, planes staged in LDS (default), 1 = in-plane stencil taps
+ * loaded directly through the vector caches, 2 = the two halves as two kernels.
+ * All produce identical results. */
 int cgfd_set_variant(cgfd_ctx *ctx, int variant);
 /* Algorithmic HBM bytes of one RK stage of this configuration (the
  * 192 B/cell + 144 B/PML-cell-axis model, FP32; doubled for FP64; 168 B/cell
