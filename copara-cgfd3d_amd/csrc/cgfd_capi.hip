@@ -250,9 +250,12 @@ static int tile_width(const cgfd_ctx *c)
 // lines, close in time; each costs its first window again (4 planes).
 // Measured at 9 / 15 / 30 planes: 200x200x150 357 / 382 / 423 us, 600x600x300
 // 4.78 / 4.81 / 4.87 ms, 32 grids of 80x80x48 per step 3.30 / 3.28 / 3.36 ms (at 9 / 15 / 25).
-// A grid that has at most 2 workgroups per CU with 1 plane each takes 1
-// (40x32x20: 15.2 -> 11.7 us); with 8 per CU 2 planes are better (64x64x64:
-// 31.2 us at 1 plane, 29.3 at 2).
+// A grid that has at most 2 workgroups per CU with 1 plane each takes 1.
+// Measured at 1 / 2 planes with the traction image, constant horizontal metrics
+// (nine): 320 workgroups, 40x32x20, 13.5 / 17.3 us (13.6 / 17.5); 576, 56x48x24,
+// 18.3 / 22.0 (18.6 / 22.2); 768, 64x64x24, 17.8 / 21.1 (18.2 / 21.5); 896, 64x64x28, 19.7 /
+// 21.8 (22.6 / 22.2); 1024, 64x64x32, 20.4 / 22.6 (24.2 / 22.8); 2048, 64x64x64, 31.8 / 29.9.
+// The line thus lies below where 1 plane stops to pay, 3 to 4 workgroups per CU.
 // The FP32 kernel that loads all nine metrics holds 3 workgroups per CU (4 with
 // constant horizontal metrics or, in 64-column tiles, a Cartesian part): a launch of 2-plane chunks just past that takes
 // 3 planes if those fit at once (64x64x64 35.4 -> 32.3 us with the traction image,
@@ -937,8 +940,9 @@ int cgfd_init(cgfd_ctx *c)
     // outputs S1 and S2 are written in every valid cell before they are read,
     // and their guard cells, zero since the allocation, never get another value
     // (600x600x300: 21 GB cleared in 5.2 ms, now half).  Where all four are
-    // cleared in the time of the further calls, up to four of ~5 us at 6 TB/s,
-    // one call per array clears them together.
+    // cleared in the time of the further calls, one call per array clears them
+    // together: a reset with all four / two cleared takes 185 / 186 us at 85 MiB in
+    // the four sets, 185 / 189 at 128, 206 / 187 at 211, 246 / 205 at 470.
     const size_t set_bytes = (size_t)NF * c->g.fs * c->esz;
     const bool all = NSETS * set_bytes <= (size_t)128 << 20;
     const size_t n = all ? NSETS : 1;

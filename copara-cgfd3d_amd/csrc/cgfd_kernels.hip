@@ -2031,8 +2031,9 @@ __global__ void record_kernel(const R *fw, long fs, const long *rlin, int nrecv,
 // every other launch of the step has read.  One workgroup, so that the counter
 // moves after all of it has read it; a launch and the gap before it less than a
 // gather and a one-lane increment (40x32x20: 74.5 -> 73.0 us per step, 64x64x64
-// replayed 155 -> 153).  Up to kRecordOne values: 400 receivers, 3780 values, were
-// slower in one workgroup (200x200x150: 1539 -> 1549 us per step).
+// replayed 155 -> 153).  Up to kRecordOne values; one launch / two, us per step of
+// 40x32x20 replayed: 108 values 53.7 / 55.0, 990 54.8 / 55.2, 1638 55.9 / 55.4, 1890
+// 56.1 / 55.2, 3420 58.4 / 55.5.
 constexpr int kRecordOne = 1024;
 template <typename R>
 __global__ void __launch_bounds__(1024) record_advance_kernel(const R *fw, long fs, const long *rlin, int nrecv,
