@@ -645,15 +645,15 @@ __global__ void __launch_bounds__(256) stage_direct_kernel(const StageArgs<R> *p
 //
 // Why two workgroups per tile and not one cell per lane: a lane that advances
 // all nine components needs 256 registers (2 wavefronts per SIMD in FP32, 1 in
-// FP64); half the components need 124-134 (FP64: 254), so 4 and 2 fit, each
+// FP64); half the components need 124-138 (FP64: 254), so 3-4 and 2 fit, each
 // wavefront has half as long a chain of instructions per plane, and a small
 // grid has twice the workgroups.  What is read twice, the metrics and in stage
 // 0 the step-start field, is read by the partner at about the same time.
-// Stage kernel, one cell per lane -> two halves: 600x600x300 5.31 -> 5.15 ms,
-// 200x200x150 428 -> 411 us, 149x131x97 with all nine metrics 171 -> 150 us,
-// 160x144x96 FP64 415 -> 313 us, 64x64x64 31.3 -> 27.8 us, 40x32x20 20.5 ->
-// 15.4 us.  With the x auxiliaries per side, the shorter chunks, the tile map
-// and the FP64 tile width they are at 4.75 ms, 352, 136, 244, 26.8 and 11.8 us.
+// Stage kernel, one cell per lane -> two halves: 600x600x300 5.31 -> 5.16 ms,
+// 200x200x150 428 -> 410 us, 149x131x97 with all nine metrics 171 -> 149 us,
+// 160x144x96 FP64 415 -> 313 us, 64x64x64 31.0 -> 27.7 us, 40x32x20 20.5 ->
+// 15.3 us.  With the layout of the x auxiliaries, the shorter chunks, the tile map
+// and the FP64 tile width they are at 4.75 ms, 353, 136, 244, 24.9 and 11.8 us.
 // Measured and not taken: both halves in one workgroup of 8
 // wavefronts that share the tile (5.24 ms, 160 us: each plane waits for the
 // slower half), the absorbing operands loaded ahead of the stencil (its
